@@ -25,7 +25,7 @@ LIB = PKG / "libsigcomp_hip.so"
 # Translation units of libsigcomp_hip.so as (source, defines): the large MLP
 # kernels are split over several units so that they compile in parallel.
 UNITS = [(CSRC / "sc_kernels.hip", ()), (CSRC / "sc_comp.hip", ()), (CSRC / "sc_gen.hip", ()),
-         (CSRC / "sc_dec_split.hip", ()),
+         (CSRC / "sc_dec_split.hip", ()), (CSRC / "sc_dec_fed.hip", ("SC_FED_RT=1",)),
          (CSRC / "sc_ctx.hip", ("SC_CTX_MODE=0",)), (CSRC / "sc_ctx.hip", ("SC_CTX_MODE=1",)),
          *[(CSRC / "sc_dec.hip", (f"SC_DEC_RT={rt}",)) for rt in range(1, 6)]]
 SOURCES = sorted({src for src, _ in UNITS})
@@ -33,7 +33,7 @@ HOST_LIB = PKG / "libsigcomp_host.so"
 HOST_SOURCES = [CSRC / "sc_host.cpp"]
 HOST_FLAGS = ["-O3", "-march=x86-64-v3", "-std=c++17", "-fPIC", "-shared", "-pthread", "-Wall", "-Wextra",
               f"-I{REPO / 'include'}"]
-HEADERS = [CSRC / "sc_device.h", CSRC / "sc_pipe.h", CSRC / "sc_kernels.h", CSRC / "sc_gen.h",
+HEADERS = [CSRC / "sc_device.h", CSRC / "sc_pipe.h", CSRC / "sc_kernels.h", CSRC / "sc_gen.h", CSRC / "sc_fed.h",
            REPO / "include" / "sigcomp_hip.h"]
 ARCH = os.environ.get("SIGCOMP_OFFLOAD_ARCH", "gfx950")
 

@@ -40,6 +40,17 @@ constexpr int64_t xch_bytes(int64_t groups) {
     return groups * XCH_GROUP + (groups * SPLIT_P_MAX * 4 + 255) / 256 * 256;
 }
 
+// Fed decode (sc_fed.h): FED_SLICES feeder workgroups per set, a set feeds
+// up to FED_SET_TILES tiles of 32 chunks (its token rings' LDS).  Exchange
+// memory per tile: the layer-0 sums (2 parities x 2 halves of the window x
+// 32 rows x 512 int32) and the token entries and step flags.
+constexpr int FED_SLICES = 16;
+constexpr int FED_SET_TILES = 20;
+constexpr int FED_SUMS = 2 * 2 * 32 * HID * 4;
+constexpr int FED_SYNC = 2 * 32 * 4 + FED_SLICES * WAVES * 4;
+constexpr int FED_MAX_TILES = 240;
+constexpr int64_t fed_bytes(int64_t tiles) { return tiles * (FED_SUMS + FED_SYNC); }
+
 // Host launchers (stream-ordered, no error check: the caller checks
 // hipGetLastError).  The MLP core follows M.pipe.
 template <int MODE>
@@ -62,6 +73,15 @@ hipError_t launch_decompress_split(const ModelDev &M, int p, unsigned groups, hi
                                    const int64_t *woff, const int32_t *wcnt, const int32_t *len, int64_t count,
                                    uint8_t *tokens, const int64_t *toff, int32_t *st, DecState *state,
                                    int32_t t_begin, int32_t t_end, uint8_t *xch, int32_t spin_max);
+
+// The fed decode of `count` chunks in `heads` workgroups of 32 RT chunks fed
+// by `sets` feeder sets (pipelined per-tensor core only): a cooperative
+// launch of heads + sets * FED_SLICES workgroups; returns its error.  `xch`
+// = fed_bytes(heads * RT) bytes, the sync part (after the sums) zeroed.
+template <int RT>
+hipError_t launch_decompress_fed(const ModelDev &M, int32_t heads, int32_t sets, hipStream_t s, const uint32_t *words,
+                                 const int64_t *woff, const int32_t *wcnt, const int32_t *len, int64_t count,
+                                 uint8_t *tokens, const int64_t *toff, int32_t *st, uint8_t *xch, int32_t spin_max);
 
 namespace {
 

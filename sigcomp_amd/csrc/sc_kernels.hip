@@ -709,7 +709,8 @@ constexpr int DEC_SEG_STEPS = 256;
 // itself (in host code the name is a stand-in, not a device address): the
 // address of the current device's copy comes from hipGetSymbolAddress.
 constexpr int64_t SCRATCH_STATE_BYTES = ((int64_t)SC_STATIC_DEC_MAX_CHUNKS * sizeof(DecState) + 255) / 256 * 256;
-constexpr int64_t SCRATCH_BYTES = SCRATCH_STATE_BYTES + 256 + xch_bytes(XCH_MAX_GROUPS);
+constexpr int64_t SCRATCH_XCH_BYTES = fed_bytes(64) > xch_bytes(XCH_MAX_GROUPS) ? fed_bytes(64) : xch_bytes(XCH_MAX_GROUPS);
+constexpr int64_t SCRATCH_BYTES = SCRATCH_STATE_BYTES + 256 + SCRATCH_XCH_BYTES;
 __device__ __align__(256) uint8_t scratch[SCRATCH_BYTES];
 
 constexpr int MAX_DEVICES = 64;
@@ -1071,12 +1072,21 @@ static int64_t dec_state_bytes(int64_t n_chunks) {
     return (n_chunks * (int64_t)sizeof(DecState) + 255) / 256 * 256;
 }
 
-// then the exchange buffers of a split launch
-static int64_t dec_xch_groups(int64_t n_chunks) { return std::min<int64_t>((n_chunks + 31) / 32, XCH_MAX_GROUPS); }
+// then the exchange buffers of a fed or split launch
+static int64_t dec_xch_bytes(int64_t n_chunks) {
+    const int64_t tiles = (n_chunks + 31) / 32;
+    return std::max(fed_bytes(std::min<int64_t>(tiles, FED_MAX_TILES)), xch_bytes(std::min<int64_t>(tiles, XCH_MAX_GROUPS)));
+}
+// What a call needs at the least (callers that sized their workspace by the
+// split decode's exchange buffers): a launch whose fed exchange does not fit
+// runs split or unsplit.
+static int64_t dec_min_bytes(int64_t n_chunks) {
+    return dec_state_bytes(n_chunks) + 256 + xch_bytes(std::min<int64_t>((n_chunks + 31) / 32, XCH_MAX_GROUPS));
+}
 
 int64_t sc_decompress_workspace_bytes(int64_t n_chunks) {
     if (n_chunks < 0) return -1;
-    return dec_state_bytes(n_chunks) + 256 + xch_bytes(dec_xch_groups(n_chunks));
+    return dec_state_bytes(n_chunks) + 256 + dec_xch_bytes(n_chunks);
 }
 
 // The launch plan's length statistics on the host (k_dec_lengths' rule):
@@ -1096,14 +1106,24 @@ static void host_len_stats(const int32_t *len, int64_t n, int64_t g0, int64_t G,
     }
 }
 
+// A fed launch: workgroups of 32 chunks, and the feeder sets beside them.
+struct FedPlan {
+    int32_t heads, sets;
+};
+constexpr int64_t FED_SET_AIM = 6;   // tiles per feeder set while CUs are free
+
+// Per-step cost of a fed launch, DEC_STEP_COST's unit: a head's chain, or
+// its set's feeders where they take longer (both measured, 2,048-token chunks).
+static int fed_step_cost(const FedPlan &f) { return std::max(222, (f.heads + f.sets - 1) / f.sets * 18); }
+
 // The decode of sc_decompress_chunks with its buffers given: `state` holds
 // DecState for n_chunks rows, `stat_dev` 4 int32 (used only when
-// lengths_host is NULL), `xch` xch_bytes(xch_groups) bytes of exchange
-// buffers for a split launch of at most xch_groups groups.
+// lengths_host is NULL), `xch` xch_cap bytes of exchange buffers for a fed
+// or split launch.
 static int decompress_run(const sc_model *m, const uint32_t *words, const int64_t *word_off, const int32_t *word_cnt,
                           const int32_t *lengths, int64_t n_chunks, uint8_t *tokens, const int64_t *tok_off,
                           int32_t *status, const int32_t *lengths_host, DecState *state, int32_t *stat_dev,
-                          uint8_t *xch, int64_t xch_groups, int32_t options, hipStream_t s) {
+                          uint8_t *xch, int64_t xch_cap, int32_t options, hipStream_t s) {
     // Under graph capture nothing may wait for the device: the launch plan
     // then needs the caller's host copy of the lengths, checked before
     // anything is enqueued so that a refused call leaves the capture valid.
@@ -1197,13 +1217,26 @@ static int decompress_run(const sc_model *m, const uint32_t *words, const int64_
     const int32_t spin_max = spin_env ? std::min(std::max(atoi(spin_env), 0), SYNC_SPIN_MAX) : SYNC_SPIN_MAX;
     auto split_p = [&](int64_t n) {   // workgroups per group of a split launch of n chunks (0: unsplit)
         const int64_t groups = (n + 31) / 32;
-        if (!split_ok || groups > std::min<int64_t>(xch_groups, XCH_MAX_GROUPS)) return 0;
+        if (!split_ok || groups > XCH_MAX_GROUPS || xch_bytes(groups) > xch_cap) return 0;
         if (split_force != 4 && groups * 8 <= cu) return 8;
         if (split_force != 8 && groups * 4 <= cu) return 4;
         return 0;
     };
+    // the fed decode (sc_fed.h) where its heads and feeder sets fit the CUs;
+    // SC_HIP_DEC_SPLIT selects the split or unsplit kernels instead
+    auto fed_plan = [&](int64_t n) {
+        FedPlan f{};
+        const int64_t tiles = (n + 31) / 32;
+        if (!split_ok || split_force >= 0 || tiles > FED_MAX_TILES || fed_bytes(tiles) > xch_cap) return f;
+        const int64_t max_sets = (cu - tiles) / FED_SLICES;
+        if (max_sets < 1 || (tiles + max_sets - 1) / max_sets > FED_SET_TILES) return f;
+        f.heads = (int32_t)tiles;
+        f.sets = (int32_t)std::min(max_sets, (tiles + FED_SET_AIM - 1) / FED_SET_AIM);
+        return f;
+    };
     const int p_left = split_p(left);
-    const int left_cost = p_left == 8 ? DEC_SPLIT_STEP_COST_P8 : p_left == 4 ? DEC_SPLIT_STEP_COST_P4 : DEC_STEP_COST[1];
+    const FedPlan f_left = fed_plan(left);
+    const int left_cost = f_left.heads ? fed_step_cost(f_left) : p_left == 8 ? DEC_SPLIT_STEP_COST_P8 : p_left == 4 ? DEC_SPLIT_STEP_COST_P4 : DEC_STEP_COST[1];
     const bool pair = can_pair && (int64_t)std::max(0, pair_max - group_max) * DEC_STEP_COST[rt_last] <
                                       (int64_t)left_max * left_cost;
     const int64_t maxlen = std::max(len_max, pair ? pair_max : 0);
@@ -1212,10 +1245,11 @@ static int decompress_run(const sc_model *m, const uint32_t *words, const int64_
         for (int rt : plan) rts += (rts.empty() ? "" : ",") + std::to_string(rt);
         const int64_t rest_last = units == 0 ? n_chunks : pair ? 0 : left;
         const int pl = rest_last ? split_p(rest_last) : 0;
-        std::fprintf(stderr, "sc_decompress_chunks: chunks %lld cu %lld plan [%s] leftover %lld %s steps %lld seg %lld\n",
+        const FedPlan fl = rest_last ? fed_plan(rest_last) : FedPlan{};
+        std::fprintf(stderr, "sc_decompress_chunks: chunks %lld cu %lld plan [%s] leftover %lld %s steps %lld seg %lld fed %d+%dx%d\n",
                      (long long)n_chunks, (long long)cu, rts.c_str(), (long long)left,
                      left == 0 ? "none" : pair ? "paired" : pl == 8 ? "split launch p8" : pl == 4 ? "split launch p4" : "launch",
-                     (long long)maxlen, (long long)seg);
+                     (long long)maxlen, (long long)seg, fl.heads, fl.sets, FED_SLICES);
     }
     int64_t start = 0;
     size_t step = 0;
@@ -1224,7 +1258,8 @@ static int decompress_run(const sc_model *m, const uint32_t *words, const int64_
         int64_t rt, count, n_second = 0;
         unsigned grid;
         int split = 0;   // workgroups per group of a split launch
-        if (step < plan.size()) {
+        const bool tail = step >= plan.size();
+        if (!tail) {
             rt = plan[step++];
             count = cu * 32 * rt;
             grid = (unsigned)cu;
@@ -1240,6 +1275,23 @@ static int decompress_run(const sc_model *m, const uint32_t *words, const int64_
         const int32_t *wcnt = word_cnt + start, *len = lengths + start;
         int32_t *st = status + start;
         DecState *ds = seg > 0 ? state + start : nullptr;
+        if (const FedPlan f = tail ? fed_plan(rest) : FedPlan{}; f.heads) {
+            hipLaunchKernelGGL(k_zero_i32, dim3(16), dim3(256), 0, s, (int32_t *)(xch + f.heads * (int64_t)FED_SUMS),
+                               f.heads * (int64_t)FED_SYNC / 4);
+            int rc = check_launch("k_zero_i32");
+            if (rc) return rc;
+            const hipError_t e = launch_decompress_fed<1>(m->dev, f.heads, f.sets, s, wds, woff, wcnt, len, count, tokens,
+                                                          toff, st, xch, spin_max);
+            if (e == hipSuccess) {
+                rc = check_launch("k_decompress_fed");
+                if (rc) return rc;
+                start += count;
+                continue;
+            }
+            (void)hipGetLastError();
+            if (e != hipErrorCooperativeLaunchTooLarge) return hip_fail(e, "k_decompress_fed");
+            split = 0;
+        }
         if (split) {
             // step flags of the grid's groups start at zero (they then hold
             // the last step each workgroup published, across segments)
@@ -1301,13 +1353,14 @@ int sc_decompress_chunks_opts(const sc_model *m, const uint32_t *words, const in
     if (n_chunks == 0) return SC_OK;
     if (!words || !word_off || !word_cnt || !lengths || !tokens || !tok_off || !status || !workspace)
         return fail(SC_ERR_ARG, "null device pointer");
-    if (workspace_bytes < sc_decompress_workspace_bytes(n_chunks)) return fail(SC_ERR_ARG, "workspace too small");
+    if (workspace_bytes < dec_min_bytes(n_chunks)) return fail(SC_ERR_ARG, "workspace too small");
     DeviceGuard guard(m->device);
     DecState *state = (DecState *)workspace;
     int32_t *stat_dev = (int32_t *)((char *)workspace + dec_state_bytes(n_chunks));
     uint8_t *xch = (uint8_t *)workspace + dec_state_bytes(n_chunks) + 256;
     return decompress_run(m, words, word_off, word_cnt, lengths, n_chunks, tokens, tok_off, status, lengths_host,
-                          state, stat_dev, xch, dec_xch_groups(n_chunks), options, as_stream(stream));
+                          state, stat_dev, xch, workspace_bytes - dec_state_bytes(n_chunks) - 256, options,
+                          as_stream(stream));
 }
 
 int sc_decompress_chunks_static(const sc_model *m, const uint32_t *words, const int64_t *word_off,
@@ -1336,7 +1389,7 @@ int sc_decompress_chunks_static(const sc_model *m, const uint32_t *words, const 
     int32_t *stat_dev = (int32_t *)((char *)base + SCRATCH_STATE_BYTES);
     uint8_t *xch = (uint8_t *)base + SCRATCH_STATE_BYTES + 256;
     return decompress_run(m, words, word_off, word_cnt, lengths, n_chunks, tokens, tok_off, status, lengths_host,
-                          state, stat_dev, xch, XCH_MAX_GROUPS, 0, as_stream(stream));
+                          state, stat_dev, xch, SCRATCH_XCH_BYTES, 0, as_stream(stream));
 }
 
 }  // extern "C"
