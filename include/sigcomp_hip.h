@@ -215,7 +215,7 @@ int sc_mfma_burn_i8(const int8_t *ops, int32_t iters, int32_t n_groups, int32_t 
 /* Bytes of device workspace sc_decompress_chunks needs for n_chunks chunks:
  * the coder state of every chunk between step segments (40 bytes per chunk),
  * the launch plan's four length statistics, and the exchange buffers of a
- * fed decode (256.5 KiB per 32 chunks, at most 240 such tiles: 60 MiB), each
+ * fed decode (128.5 KiB per 32 chunks, at most 256 such tiles: 32 MiB), each
  * part 256-byte aligned.  sc_decompress_chunks also takes less, down to 32
  * KiB + 32 bytes per 32 chunks (at most 64) after the other parts: launches
  * whose fed exchange does not fit then run split (4 or 8 workgroups per 32
@@ -241,9 +241,10 @@ int64_t sc_decompress_workspace_bytes(int64_t n_chunks);
  * descending length (as QuantMLPCompression passes them) give the shortest
  * schedule: the shortest chunks are then left over after the full waves of
  * workgroups and follow the shortest chunks of the last full wave in the
- * same rows.  A launch of up to 140 tiles of 32 chunks (on 256 CUs) runs fed:
- * one workgroup per tile decodes it, sets of 16 more compute layer 0 of the
- * next step for up to 20 tiles each, and they wait for each other every step
+ * same rows.  A launch of at most 256 tiles of 32 chunks (on 256 CUs) runs
+ * fed: one workgroup per tile or pair of tiles decodes it, sets of 16 more
+ * compute layer 0 of the next step for up to 32 tiles each, and they wait for
+ * each other every step
  * (a cooperative launch, so all are resident; a bounded wait,
  * SC_STATUS_SYNC_TIMEOUT when it expires), except
  * on a stream under graph capture.  Replaces
@@ -274,7 +275,7 @@ int sc_decompress_chunks_opts(const sc_model *model, const uint32_t *words, cons
  * forbid hipMalloc).  sc_decompress_chunks with its workspace replaced by a
  * static device array the library holds on each GPU it runs on until the
  * process ends (SC_STATIC_DEC_MAX_CHUNKS chunks of coder state and the
- * exchange buffers of a fed decode of 64 tiles, 18.5 MiB; a larger leftover
+ * exchange buffers of a fed decode of 128 tiles, 18.6 MiB; a larger leftover
  * launch runs unsplit);
  * the call allocates nothing.  n_chunks above SC_STATIC_DEC_MAX_CHUNKS ->
  * SC_ERR_ARG.  Every call on one GPU shares that GPU's array: calls that

@@ -8,21 +8,29 @@
 // other 63 are known a whole step earlier.  So the work is split by role:
 //
 //   * a HEAD workgroup owns 32 RT chunks.  Per step it adds the newest
-//     token's position (64 KB of weights, held in registers) to layer-0 sums
+//     token's position (64 KB of weights, held on chip) to layer-0 sums
 //     that are already there, runs the hidden and output layers (2 MB
-//     streamed per step from its XCD's L2) and the decoder step, and
-//     publishes the step's 32 RT tokens;
+//     streamed per step from its XCD's L2; at RT = 1 the output layer's 128
+//     KB are held in registers) and the decoder step, and publishes the
+//     step's 32 RT tokens;
 //   * FED_SLICES FEEDER workgroups form a set that computes those sums for up
-//     to FED_SET_TILES tiles of 32 chunks.  Each feeder keeps 1/16 of layer 0
-//     (two n-tiles over half of the window, 256 KB) in its registers for
-//     the whole decode, so the sums of a tile cost it 64 MFMAs per wave and
-//     no weight traffic: waves take eight positions each, their partial
-//     sums meet in LDS, and the int32 sums (both halves of the window
-//     separately, the head adds them) go to the exchange buffer.
+//     to FED_SET_TILES tiles of 32 chunks.  Each feeder keeps one n-tile of
+//     layer 0 (256 KB, its four waves 16 window positions each) in its
+//     registers for the whole decode, so the sums of a tile cost it 64 MFMAs
+//     per wave and no weight traffic; the waves' partial sums meet in LDS
+//     and go to the exchange buffer.
+//
+// Measured per step at 2,048-token chunks: a 32-row head 20.1 us (layers 1-6
+// 12.1, the last hidden layer 2.3, the output layer 1.2, the decoder step
+// 2.5, layer 0's last position 1.4; 22.2 with the output layer streamed and
+// the window's halves summed by the head), a 64-row head 31, a tile at its
+// feeders 1.73 (1.3 of it products and operand reads, bound by the LDS: each
+// operand fragment feeds one MFMA; two n-tiles over half of the window per
+// feeder read half as much, 0.95, but double the sums that a head loads).
 //
 // While a head runs step t + 1 its feeders compute the sums of step t + 2, so
 // the exchange's latency (~1.5 us each way) is off the chain, and a head's
-// step is the hidden layers' L1 time plus the decoder step.
+// step is the hidden layers' L1 time (64 B/clock) plus the decoder step.
 //
 // Exchange of one tile (fed_bytes): two parity buffers of sums, two parity
 // rows of 32 token entries, FED_SLICES * WAVES step flags.  The sums of step
@@ -47,14 +55,14 @@
 namespace sc {
 namespace {
 
-constexpr int FED_POS = WIN / 2 / WAVES;             // window positions per feeder wave
+constexpr int FED_POS = WIN / WAVES;                 // window positions per feeder wave
 constexpr int FED_KS = EDIM / 32;                    // k-steps per position
 
-// feeder LDS: embedding table, partial sums (2 parities x 4 waves x 8 KB),
+// feeder LDS: embedding table, partial sums (2 parities x 4 waves x 4 KB),
 // token rings, step counts
 constexpr int FED_RED_OFF = EMB_BYTES;
-constexpr int FED_RED_WAVE = 2 * 4 * 64;   // 16-byte pieces of a wave's two tiles
-constexpr int FED_RED_BYTES = 2 * WAVES * FED_RED_WAVE * 16;
+constexpr int FED_RED_BYTES = 2 * WAVES * 4 * 64 * 16;
+constexpr int RED_READ = 5;   // position whose region reads the partial sums (a barrier before it)
 constexpr int FED_TOK_OFF = FED_RED_OFF + FED_RED_BYTES;
 constexpr int FED_STEPS_OFF = FED_TOK_OFF + FED_SET_TILES * WIN * 32;
 constexpr int FED_FEEDER_LDS = FED_STEPS_OFF + FED_SET_TILES * 4;
@@ -83,7 +91,15 @@ struct FedHeadLds {
     static constexpr int RING = WBUF_OFF + R * WBUF * 4;
     static constexpr int LAST = RING + R * WIN;
     static constexpr int MISC = LAST + R * 2;
-    static constexpr int BYTES = MISC + 8;
+    // layer 0's last position, [n-tile][k-step] fragments (RES)
+    static constexpr int WLAST = (MISC + 8 + 15) / 16 * 16;
+    // RES: a 32-row head keeps the output layer in registers and layer 0's
+    // last position in LDS; a 64-row head has neither to spare (twice the
+    // accumulators and rows) and gains less: its products take as long as
+    // the weight stream.
+    static constexpr bool RES = RT == 1;
+    static constexpr int BYTES = WLAST + (RES ? HID / 32 * FED_KS * 1024 : 0);
+    static_assert(BYTES <= 160 * 1024, "LDS of a CU");
     static_assert(ACT % 16 == 0 && PAR % 16 == 0 && SLOT % 16 == 0 && LUT % 16 == 0 && MISC % 8 == 0, "alignment");
 };
 
@@ -167,13 +183,11 @@ __device__ __forceinline__ void fed_decode_rows(const FedRows &c, uint32_t *slot
 __device__ __forceinline__ uint32_t *fed_sync(uint8_t *xch, int tiles, int tile) {
     return (uint32_t *)(xch + (int64_t)tiles * FED_SUMS + (int64_t)tile * FED_SYNC);
 }
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t fed_sums(uint8_t *xch, int tile) {
-    return __builtin_amdgcn_make_buffer_rsrc((void *)(xch + (int64_t)tile * FED_SUMS), (short)0, FED_SUMS, 0x00020000);
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t fed_sums(uint8_t *xch, int tile, int bytes = FED_SUMS) {
+    return __builtin_amdgcn_make_buffer_rsrc((void *)(xch + (int64_t)tile * FED_SUMS), (short)0, bytes, 0x00020000);
 }
 // byte offset of n-tile nt's sums (4 KB: register quarter e at e * 1024 + lane * 16)
-__device__ __forceinline__ int fed_sums_off(int step, int half, int nt) {
-    return (((step & 1) * 2 + half) * (HID / 32) + nt) * 4096;
-}
+__device__ __forceinline__ int fed_sums_off(int step, int nt) { return ((step & 1) * (HID / 32) + nt) * 4096; }
 
 // ---- feeder ------------------------------------------------------------
 __device__ __forceinline__ void fed_feeder(const ModelDev &M, uint8_t *s_mem, const int32_t *__restrict__ lengths,
@@ -196,158 +210,228 @@ __device__ __forceinline__ void fed_feeder(const ModelDev &M, uint8_t *s_mem, co
         const int64_t c = (int64_t)((set + j * sets) / rt) * (32 * rt) + i % (32 * rt);
         if (c < n_chunks) atomicMax(&s_steps[j], lengths[c]);
     }
-    // this wave's weights, in registers for the whole decode: n-tiles 2 np
-    // and 2 np + 1 over positions p0 .. p0 + 7.  The window's last position
-    // is the head's: zero here, so its slot may hold any token.
-    const int half = slice & 1, np = slice >> 1;
-    const int p0 = half * (WIN / 2) + wave * FED_POS;
+    // this wave's weights, in registers for the whole decode: n-tile `slice`
+    // over positions p0 .. p0 + 15.  The window's last position is the
+    // head's: zero here, so its slot may hold any token.
+    const int p0 = wave * FED_POS;
     const int g = lane >> 5, rl = lane & 31, kg = g << 4, voff = lane * 16;
-    v4i w[FED_POS][FED_KS][2];
-    v4i bias[2] = {};   // of the sums this wave owns (below), in the window's first half only
+    v4i w[FED_POS][FED_KS];
+    v4i bias;   // of the sums this wave owns (below)
     {
         const __amdgpu_buffer_rsrc_t rs = layer_rsrc(M.layer[0]);
 #pragma unroll
         for (int i = 0; i < FED_POS; ++i)
 #pragma unroll
-            for (int q = 0; q < FED_KS; ++q)
+            for (int q = 0; q < FED_KS; ++q) {
+                w[i][q] = wload_s(rs, voff, (slice * KT0 + (p0 + i) * FED_KS + q) * 1024);
+                if (i == FED_POS - 1 && wave == WAVES - 1) w[i][q] = v4i{0, 0, 0, 0};
+            }
 #pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    w[i][q][j] = wload_s(rs, voff, ((2 * np + j) * KT0 + (p0 + i) * FED_KS + q) * 1024);
-                    if (p0 + i == WIN - 1) w[i][q][j] = v4i{0, 0, 0, 0};
-                }
-        if (half == 0) {
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-#pragma unroll
-                for (int k = 0; k < 4; ++k)   // register v of a tile: feature 8 (v / 4) + 4 g + v % 4
-                    bias[h][k] = (int)M.layer[0].par[(2 * np + (wave >> 1)) * PAR_DWORDS +
-                                                     8 * (2 * (wave & 1) + h) + 4 * g + k];
-        }
+        for (int k = 0; k < 4; ++k)   // register v of a tile: feature 8 (v / 4) + 4 g + v % 4
+            bias[k] = (int)M.layer[0].par[slice * PAR_DWORDS + 8 * wave + 4 * g + k];
     }
     __syncthreads();
+    const int steps_l = lane < mine ? s_steps[lane] : 0;   // lane j: steps of the set's tile j
     int maxs = 0;
-    for (int j = 0; j < mine; ++j) maxs = max(maxs, __builtin_amdgcn_readfirstlane(s_steps[j]));
+    for (int j = 0; j < mine; ++j) maxs = max(maxs, __builtin_amdgcn_readlane(steps_l, j));
     // items (tile j, step s) in step order; steps past a tile's end are skipped
-    auto next = [&](int &j, int &s) {
-        for (;;) {
-            if (++j >= mine) {
-                j = 0;
-                ++s;
-            }
-            if (s >= maxs) return false;
-            if (s < __builtin_amdgcn_readfirstlane(s_steps[j])) return true;
-        }
+    auto next = [&](int &j, int &s) __attribute__((always_inline)) {
+        do {
+            const bool wrap = ++j >= mine;
+            j = wrap ? 0 : j;
+            s += wrap;
+        } while (__builtin_expect(s < maxs && s >= __builtin_amdgcn_readlane(steps_l, j), 0));
+        return s < maxs;
     };
-    auto entry_at = [&](int j, int s) {   // the token entries that the sums of step s wait for
-        return fed_sync(xch, tiles, set + j * sets) + ((s - 2) & 1) * 32 + rl;
+    // the token entries that the sums of step s wait for
+    const char *ent0 = (const char *)fed_sync(xch, tiles, set) + rl * 4;
+    auto load_entries = [&](int j, int s) {
+        return __hip_atomic_load((const uint32_t *)(ent0 + (uint32_t)(j * sets * FED_SYNC + (s & 1) * 128)),
+                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     };
     bool dead = false;
-    int32_t *pend = nullptr;   // flag of the item whose stores are in flight
-    int32_t pend_v = 0;
-    auto publish = [&] {
-        if (pend) {
-            wait_counts<0, 15>();
-            if (lane == 0 && !dead) __hip_atomic_store(pend, pend_v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            pend = nullptr;
-        }
+    // The last item's reduction: wave v sums register quarter v of the tile
+    // over the four waves.  It runs beside the next item's products when
+    // that item is ready, else at once (finish) before the wave polls; one
+    // barrier per item either way.  s_red has two parities: a wave writes a
+    // parity again only after the next item's barrier, which every reader of
+    // this one has reached.
+    v16i prev = {};
+    bool open = false;                  // the last item's reduction is still to do
+    int par = 0, poff = 0, pval = 0;    // its parity, sums offset and flag value
+    int32_t *pflag = nullptr;
+    int ptile = set;
+    auto red_at = [&](int w_, int e) { return s_red + ((par * WAVES + w_) * 4 + e) * 64 + lane; };
+    auto red_put = [&](int e) __attribute__((always_inline)) {
+        *red_at(wave, e) = v4i{prev[4 * e], prev[4 * e + 1], prev[4 * e + 2], prev[4 * e + 3]};
+    };
+    auto announce = [&] {   // the wave's stores have completed
+        wait_counts<0, 15>();
+        if (lane == 0 && !dead) __hip_atomic_store(pflag, pval, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    auto finish = [&] {
+        if (!open) return;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) red_put(e);
+        __syncthreads();
+        v4u x = (v4u)bias;
+#pragma unroll
+        for (int f = 0; f < WAVES; ++f) x += (v4u)*red_at(f, wave);
+        __builtin_amdgcn_raw_buffer_store_b128(x, fed_sums(xch, ptile), voff, poff, CPOL_SC1);
+        announce();
+        open = false;
+    };
+    auto tok_at = [&](int j, int s, int i) {   // slot of window position p0 + i of step s: token s - 64 + p0 + i
+        return s_tok + (j * WIN + ((s + p0 + i) & (WIN - 1))) * 32 + rl;
     };
     uint32_t ent = 0;
-    int j = -1, s = 0, par = 0;
+    int j = -1, s = 0;
     bool have = next(j, s);
+    int ea[FED_POS];   // the item's table addresses
+#pragma unroll
+    for (int i = 0; i < FED_POS; ++i) ea[i] = emb_off(SOS, 0) + kg;
     while (have) {
+        // (pinned: half of the weights in accumulation registers, from which
+        // an MFMA can read them, instead of copies before each use)
+#pragma unroll
+        for (int i = 0; i < FED_POS; ++i)
+#pragma unroll
+            for (int q = 0; q < FED_KS; ++q) {
+                if (i >= FED_POS / 2) asm volatile("" : "+a"(w[i][q]));
+                else asm volatile("" : "+v"(w[i][q]));
+            }
         int jn = j, sn = s;
         const bool more = next(jn, sn);
-        if (s >= 2) {
+        if (__builtin_expect(s >= 2, 1)) {
             const uint32_t want = (uint32_t)(s - 1) & 0xFFFFFFu;
-            if (!dead && __builtin_amdgcn_ballot_w64((ent >> 8) != want) != 0) {
-                publish();   // nothing may wait for this item while its head waits for the last one
-                const uint32_t *src = entry_at(j, s);
+            if (__builtin_expect(!dead && __builtin_amdgcn_ballot_w64((ent >> 8) != want) != 0, 0)) {
+                finish();   // this item's head may be waiting for the last item
                 for (int n = 0;; ++n) {
                     if (n >= spin_max) {
                         dead = true;
                         break;
                     }
-                    ent = __hip_atomic_load(src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    ent = load_entries(j, s);
                     if (__builtin_amdgcn_ballot_w64((ent >> 8) != want) == 0) break;
                     __builtin_amdgcn_s_sleep(2);
                 }
             }
             // every wave writes the tile's tokens (the same bytes) and reads
             // only after its own writes: no barrier
-            s_tok[(j * WIN + ((s - 2) & (WIN - 1))) * 32 + rl] = (uint8_t)ent;
+            *tok_at(j, s, WIN - 2 - p0) = (uint8_t)ent;
+            // the newest token's position was not yet known when the
+            // addresses were prepared
+            if (p0 + FED_POS == WIN) ea[FED_POS - 2] = emb_off((int)(ent & 0xFF), 0) + kg;
         }
         // the next item's tokens travel beside this item's products
-        ent = more && sn >= 2 ? __hip_atomic_load(entry_at(jn, sn), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
-        // addresses of the eight positions, then a position's four operand
-        // fragments are read while the previous position's products run
-        int tok[FED_POS], ea[FED_POS];
-#pragma unroll
-        for (int i = 0; i < FED_POS; ++i)   // slot of token s - 64 + p
-            tok[i] = (int)s_tok[(j * WIN + ((s + p0 + i) & (WIN - 1))) * 32 + rl];
-        // (read either way: a select, no branch per position)
-        asm volatile("" : "+v"(tok[0]), "+v"(tok[1]), "+v"(tok[2]), "+v"(tok[3]), "+v"(tok[4]), "+v"(tok[5]),
-                     "+v"(tok[6]), "+v"(tok[7]));
-#pragma unroll
-        for (int i = 0; i < FED_POS; ++i) ea[i] = emb_off(s + p0 + i < WIN ? SOS : tok[i], 0) + kg;
+        // (unused if it is none or its step < 2)
+        ent = load_entries(jn, sn);
         v4i b[2][FED_KS];
 #pragma unroll
         for (int q = 0; q < FED_KS; ++q) b[0][q] = *(const v4i *)(s_emb + ea[0] + q * 32);
-        v16i acc[2] = {v16i{}, v16i{}};
+        v16i acc[2] = {v16i{}, v16i{}};   // two chains: one would wait for itself
+        int tn[FED_POS];
+        v4u part[WAVES];
+        // (a reduction that finish() has done is repeated without its
+        // barrier and stored nowhere)
+        const __amdgpu_buffer_rsrc_t rs_open = fed_sums(xch, __builtin_amdgcn_readfirstlane(ptile),
+                                                        __builtin_amdgcn_readfirstlane(open ? FED_SUMS : 0));
+        const int off_open = __builtin_amdgcn_readfirstlane(poff);
         __builtin_amdgcn_sched_barrier(0);
+        // One position per region: its products, the next position's operand
+        // reads, the next item's address of this position, and a piece of
+        // the last item's reduction.
         static_for<FED_POS>([&](auto ic) __attribute__((always_inline)) {
             constexpr int i = decltype(ic)::value;
             if constexpr (i + 1 < FED_POS) {
 #pragma unroll
                 for (int q = 0; q < FED_KS; ++q) b[(i + 1) & 1][q] = *(const v4i *)(s_emb + ea[i + 1] + q * 32);
             }
+            tn[i] = (int)*tok_at(jn, sn, i);
+            if constexpr (i > 0) {
+                ea[i - 1] = emb_off(sn + p0 + i - 1 < WIN ? SOS : tn[i - 1], 0) + kg;
+                asm volatile("" : "+v"(ea[i - 1]));   // here, not after the last product
+
+            }
+            if constexpr (i < 4) red_put(i);
+            if constexpr (i == RED_READ) {
+#pragma unroll
+                for (int f = 0; f < WAVES; ++f) part[f] = (v4u)*red_at(f, wave);
+            }
+            if constexpr (i == RED_READ + 1)
+                __builtin_amdgcn_raw_buffer_store_b128((v4u)bias + part[0] + part[1] + part[2] + part[3], rs_open, voff,
+                                                       off_open, CPOL_SC1);
 #pragma unroll
             for (int q = 0; q < FED_KS; ++q)
-#pragma unroll
-                for (int x = 0; x < 2; ++x)
-                    acc[x] = __builtin_amdgcn_mfma_i32_32x32x32_i8(w[i][q][x], b[i & 1][q], acc[x], 0, 0, 0);
-            static_for<2 * FED_KS>([&](auto mc) __attribute__((always_inline)) {
-                if constexpr (i + 1 < FED_POS && decltype(mc)::value < FED_KS) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                acc[q & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(w[i][q], b[i & 1][q], acc[q & 1], 0, 0, 0);
+            static_for<FED_KS>([&](auto) __attribute__((always_inline)) {
+                __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);   // LDS reads
+                __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);   // LDS writes
+                __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);   // VALU
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // MFMA
             });
             __builtin_amdgcn_sched_barrier(0);
+            if constexpr (i == RED_READ - 1) {
+                if (open) __syncthreads();
+            }
         });
-        publish();   // the previous item's stores have had the products' time to complete
-        // Wave v sums registers 8 (v & 1) .. + 7 of n-tile v >> 1 over the four
-        // waves (two parities of s_red, so one barrier per item: a wave
-        // writes a parity again only after the next item's barrier, which
-        // every reader of this one has reached).
-        v4i *red = s_red + par * (WAVES * FED_RED_WAVE) + lane;
+        ea[FED_POS - 1] = emb_off(sn + p0 + FED_POS - 1 < WIN ? SOS : tn[FED_POS - 1], 0) + kg;
+        if (open) announce();   // the store has had eight positions' time
+        prev = acc[0] + acc[1];
+        open = true;
         par ^= 1;
-#pragma unroll
-        for (int x = 0; x < 2; ++x)
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                red[wave * FED_RED_WAVE + (x * 4 + e) * 64] =
-                    v4i{acc[x][4 * e], acc[x][4 * e + 1], acc[x][4 * e + 2], acc[x][4 * e + 3]};
-        __syncthreads();
-        const int T = set + j * sets;
-        const __amdgpu_buffer_rsrc_t rs = fed_sums(xch, T);
-        {
-            v4u x[2] = {(v4u)bias[0], (v4u)bias[1]};
-#pragma unroll
-            for (int f = 0; f < WAVES; ++f)
-#pragma unroll
-                for (int h = 0; h < 2; ++h) x[h] += (v4u)red[f * FED_RED_WAVE + (2 * wave + h) * 64];
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-                __builtin_amdgcn_raw_buffer_store_b128(
-                    x[h], rs, voff, fed_sums_off(s, half, 2 * np + (wave >> 1)) + (2 * (wave & 1) + h) * 1024, CPOL_SC1);
-        }
-        pend = (int32_t *)fed_sync(xch, tiles, T) + 64 + slice * WAVES + wave;
-        pend_v = s + 1;
+        poff = fed_sums_off(s, slice) + wave * 1024;
+        pval = s + 1;
+        ptile = set + j * sets;
+        pflag = (int32_t *)fed_sync(xch, tiles, ptile) + 64 + slice * WAVES + wave;
         j = jn;
         s = sn;
         have = more;
     }
-    publish();
+    finish();
 }
 
 // ---- head --------------------------------------------------------------
+
+// The output layer with its weights in registers (wo[k-step][n-tile]): as
+// pipe_hidden with LASTL (entry and exit conditions), without weight loads.
+template <int RT>
+__device__ __forceinline__ void fed_output(const LayerDev &Lp, const LayerDev &L, uint8_t *s_act, uint32_t *s_parw,
+                                           int l, v16i (&accA)[PNT][RT], v16i (&accB)[PNT][RT],
+                                           const v4i (&wo)[KTH][PNT], uint32_t (&pk)[PNT][RT][4], int wave, int lane) {
+    constexpr int MF = PNT * RT, BLK = Slot<true>::BLK;
+    const int g = lane >> 5, bbase = pact_off(lane & 31, g);
+    const uint32_t *cur0 = s_parw + slot_p0(l) * BLK;
+    v4i b[2][RT];
+    read_b<RT>(s_act, bbase, 0, b[0]);
+    const RqUni up = rq_uni(Lp);
+    v16i bias[PNT];
+#pragma unroll
+    for (int j = 0; j < PNT; ++j) bias[j] = bias_tile<true>(cur0, j, g);
+    static_for<KTH>([&](auto vc) __attribute__((always_inline)) {
+        constexpr int v = decltype(vc)::value;
+        if constexpr (v != 7 && v != KTH - 1) read_b<RT>(s_act, bbase, v + 1, b[(v + 1) & 1]);
+        if constexpr (v < 8) rq_words_uni<true, 0, RT>(accB[v / 4], v % 4, up, pk[v / 4]);
+#pragma unroll
+        for (int j = 0; j < PNT; ++j)
+#pragma unroll
+            for (int i = 0; i < RT; ++i)
+                accA[j][i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wo[v][j], b[v & 1][i], v == 0 ? bias[j] : accA[j][i],
+                                                                   0, 0, 0);
+        pipe_schedule<MF, (v != 7 && v != KTH - 1 ? RT : 0), 0, (v < 8 ? 12 : 0)>();
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (v == 7) {
+            pstore_perm<RT>(pk, 8 + 2 * wave, s_act, lane);
+            __syncthreads();
+            read_b<RT>(s_act, bbase, 8, b[0]);
+        }
+    });
+    rq_pass_uni<false, RT>(accA, rq_uni(L), pk);
+    __syncthreads();
+    pstore_natural<RT>(pk, 2 * wave, s_act, lane);
+    __syncthreads();
+}
+
 template <int RT>
 __device__ __forceinline__ void fed_head(const ModelDev &M, uint8_t *s_mem, const uint32_t *__restrict__ words,
                                          const int64_t *__restrict__ word_off, const int32_t *__restrict__ word_cnt,
@@ -429,15 +513,30 @@ __device__ __forceinline__ void fed_head(const ModelDev &M, uint8_t *s_mem, cons
     uint32_t *s_parw = s_par + wave * PIPE_SLOTS * BLK;
     constexpr int PPD = ppd<RT>();
     auto ntile = [&](int j) { return j < PNT ? nb0 + j : nb1 + j - PNT; };
-    // layer 0's last window position for the wave's four n-tiles
-    v4i wlast[2 * PNT][FED_KS];
+    // layer 0's last window position for the wave's four n-tiles (RES: the
+    // wave's own 16 KB of LDS)
+    constexpr bool RES = H::RES;
+    v4i *s_wlast = (v4i *)(s_mem + H::WLAST) + wave * (2 * PNT * FED_KS * 64) + lane;
+    v4i wlast[RES ? 1 : 2 * PNT][FED_KS];
     {
         const __amdgpu_buffer_rsrc_t rs0 = layer_rsrc(M.layer[0]);
 #pragma unroll
         for (int j = 0; j < 2 * PNT; ++j)
 #pragma unroll
-            for (int q = 0; q < FED_KS; ++q)
-                wlast[j][q] = wload_s(rs0, voff, (ntile(j) * KT0 + (WIN - 1) * FED_KS + q) * 1024);
+            for (int q = 0; q < FED_KS; ++q) {
+                const v4i x = wload_s(rs0, voff, (ntile(j) * KT0 + (WIN - 1) * FED_KS + q) * 1024);
+                if constexpr (RES) s_wlast[(j * FED_KS + q) * 64] = x;
+                else wlast[j][q] = x;
+            }
+    }
+    const int last = M.n_layers - 1;   // at least 3 (the launch's rule)
+    v4i wo[RES ? KTH : 1][PNT];        // RES: the output layer's weights
+    if constexpr (RES) {
+        const __amdgpu_buffer_rsrc_t rso = layer_rsrc(M.layer[last]);
+#pragma unroll
+        for (int q = 0; q < KTH; ++q)
+#pragma unroll
+            for (int j = 0; j < PNT; ++j) wo[q][j] = wload_s(rso, voff, ((nb0 + j) * KTH + q) * 1024);
     }
     bool dead = false;
     int32_t fl[RT];   // this lane's feeder flag of each tile
@@ -449,9 +548,9 @@ __device__ __forceinline__ void fed_head(const ModelDev &M, uint8_t *s_mem, cons
             fl[i] = __hip_atomic_load((int32_t *)fed_sync(xch, tiles, head * RT + i) + 64 + lane, __ATOMIC_RELAXED,
                                       __HIP_MEMORY_SCOPE_AGENT);
     };
-    v4i px[RT][2][2 * PNT][4];
-    // the sums of step s: wait for the feeders, then issue the loads
-    auto fetch_sums = [&](int32_t s) __attribute__((always_inline)) {
+    v4i px[RT][2 * PNT][4];   // the next step's sums
+    // waits for the feeders' sums of step s
+    auto wait_sums = [&](int32_t s) __attribute__((always_inline)) {
         auto late = [&] {
             bool l = false;
 #pragma unroll
@@ -470,24 +569,33 @@ __device__ __forceinline__ void fed_head(const ModelDev &M, uint8_t *s_mem, cons
                 __builtin_amdgcn_s_sleep(2);
             }
         }
+    };
+    auto load_sums = [&](int32_t s) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < RT; ++i) {
             const __amdgpu_buffer_rsrc_t rs = fed_sums(xch, head * RT + i);
 #pragma unroll
-            for (int h = 0; h < 2; ++h)
+            for (int j = 0; j < 2 * PNT; ++j)
 #pragma unroll
-                for (int j = 0; j < 2 * PNT; ++j)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        px[i][h][j][e] = (v4i)__builtin_amdgcn_raw_buffer_load_b128(
-                            rs, voff, fed_sums_off(s, h, ntile(j)) + e * 1024, CPOL_SC1);
+                for (int e = 0; e < 4; ++e)
+                    px[i][j][e] = (v4i)__builtin_amdgcn_raw_buffer_load_b128(rs, voff, fed_sums_off(s, ntile(j)) + e * 1024,
+                                                                             CPOL_SC1);
         }
     };
-    const int last = M.n_layers - 1;
     const RqUni u0 = rq_uni(M.layer[0]);
-    if (steps > 0) fetch_sums(0);
+    if (steps > 0) {
+        wait_sums(0);
+        load_sums(0);
+    }
 #pragma unroll 1
     for (int32_t t = 0; t < steps; ++t) {
+        // (the output layer's weights stay in the accumulation registers)
+        if constexpr (RES) {
+#pragma unroll
+            for (int q = 0; q < KTH; ++q)
+#pragma unroll
+                for (int j = 0; j < PNT; ++j) asm volatile("" : "+a"(wo[q][j]));
+        }
         v16i accA[PNT][RT], accB[PNT][RT];
         v4i w[2][PPD][PNT];
         uint32_t pk[PNT][RT][4];
@@ -512,11 +620,14 @@ __device__ __forceinline__ void fed_head(const ModelDev &M, uint8_t *s_mem, cons
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
 #pragma unroll
-                        for (int k = 0; k < 4; ++k)
-                            a[4 * e + k] = (int)((uint32_t)px[i][0][j][e][k] + (uint32_t)px[i][1][j][e][k]);
+                        for (int k = 0; k < 4; ++k) a[4 * e + k] = px[i][j][e][k];
 #pragma unroll
-                    for (int q = 0; q < FED_KS; ++q)
-                        a = __builtin_amdgcn_mfma_i32_32x32x32_i8(wlast[j][q], b[q], a, 0, 0, 0);
+                    for (int q = 0; q < FED_KS; ++q) {
+                        v4i wl;
+                        if constexpr (RES) wl = s_wlast[(j * FED_KS + q) * 64];
+                        else wl = wlast[j][q];
+                        a = __builtin_amdgcn_mfma_i32_32x32x32_i8(wl, b[q], a, 0, 0, 0);
+                    }
                 }
             }
             par_put<UNI>(s_parw + slot_p0(1) * BLK, prn, lane);
@@ -526,23 +637,31 @@ __device__ __forceinline__ void fed_head(const ModelDev &M, uint8_t *s_mem, cons
             pstore_perm<RT>(pk, nb1, s_act, lane);
             __syncthreads();
         }
-        if (last == 1) {
-            load_flags();
-            pipe_hidden<RT, true, UNI, true>(M.layer[0], M.layer[1], M.layer[1], s_act, s_parw, 1, accA, accB, w, pk,
-                                             wave, lane);
-        } else {
-            pipe_hidden<RT, false, UNI, true>(M.layer[0], M.layer[1], M.layer[2], s_act, s_parw, 1, accA, accB, w, pk,
-                                              wave, lane);
+        pipe_hidden<RT, false, UNI, true>(M.layer[0], M.layer[1], M.layer[2], s_act, s_parw, 1, accA, accB, w, pk,
+                                          wave, lane);
 #pragma unroll 1
-            for (int l = 2; l < last; ++l)
-                pipe_hidden<RT, false, UNI>(M.layer[l - 1], M.layer[l], M.layer[l + 1], s_act, s_parw, l, accA, accB,
-                                            w, pk, wave, lane);
-            load_flags();   // read back behind the output layer
-            pipe_hidden<RT, true, UNI>(M.layer[last - 1], M.layer[last], M.layer[last], s_act, s_parw, last, accA,
-                                       accB, w, pk, wave, lane);
+        for (int l = 2; l < last - 1; ++l)
+            pipe_hidden<RT, false, UNI>(M.layer[l - 1], M.layer[l], M.layer[l + 1], s_act, s_parw, l, accA, accB, w,
+                                        pk, wave, lane);
+        load_flags();   // read back behind the last hidden layer
+        pipe_hidden<RT, false, UNI, false, false, !RES>(M.layer[last - 2], M.layer[last - 1], M.layer[last], s_act,
+                                                        s_parw, last - 1, accA, accB, w, pk, wave, lane);
+        if constexpr (RES) {
+            // the next step's sums travel beside the output layer, which
+            // leaves the CU's vector L1 idle
+            if (t + 1 < steps) {
+                wait_sums(t + 1);
+                load_sums(t + 1);
+            }
+            fed_output<RT>(M.layer[last - 1], M.layer[last], s_act, s_parw, last, accA, accB, wo, pk, wave, lane);
+        } else {
+            pipe_hidden<RT, true, UNI>(M.layer[last - 1], M.layer[last], M.layer[last], s_act, s_parw, last, accA, accB,
+                                       w, pk, wave, lane);
+            if (t + 1 < steps) {
+                wait_sums(t + 1);
+                load_sums(t + 1);
+            }
         }
-        // the next step's sums travel beside the decoder step
-        if (t + 1 < steps) fetch_sums(t + 1);
 #pragma unroll 1
         for (int gi = wave; gi < R / 4; gi += 2 * WAVES) {
             // groups of four rows whose chunks have all ended cost nothing

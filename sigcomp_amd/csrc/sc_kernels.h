@@ -42,13 +42,13 @@ constexpr int64_t xch_bytes(int64_t groups) {
 
 // Fed decode (sc_fed.h): FED_SLICES feeder workgroups per set, a set feeds
 // up to FED_SET_TILES tiles of 32 chunks (its token rings' LDS).  Exchange
-// memory per tile: the layer-0 sums (2 parities x 2 halves of the window x
-// 32 rows x 512 int32) and the token entries and step flags.
+// memory per tile: the layer-0 sums (2 parities x 32 rows x 512 int32) and the token entries and step flags.
 constexpr int FED_SLICES = 16;
-constexpr int FED_SET_TILES = 20;
-constexpr int FED_SUMS = 2 * 2 * 32 * HID * 4;
+constexpr int FED_SET_TILES = 32;
+constexpr int FED_SUMS = 2 * 32 * HID * 4;
 constexpr int FED_SYNC = 2 * 32 * 4 + FED_SLICES * WAVES * 4;
-constexpr int FED_MAX_TILES = 240;
+constexpr int FED_MAX_TILES = 256;
+constexpr int FED_MIN_LAYERS = 4;   // a first, a last hidden and an output layer after layer 0
 constexpr int64_t fed_bytes(int64_t tiles) { return tiles * (FED_SUMS + FED_SYNC); }
 
 // Host launchers (stream-ordered, no error check: the caller checks

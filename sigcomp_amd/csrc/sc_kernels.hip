@@ -709,7 +709,8 @@ constexpr int DEC_SEG_STEPS = 256;
 // itself (in host code the name is a stand-in, not a device address): the
 // address of the current device's copy comes from hipGetSymbolAddress.
 constexpr int64_t SCRATCH_STATE_BYTES = ((int64_t)SC_STATIC_DEC_MAX_CHUNKS * sizeof(DecState) + 255) / 256 * 256;
-constexpr int64_t SCRATCH_XCH_BYTES = fed_bytes(64) > xch_bytes(XCH_MAX_GROUPS) ? fed_bytes(64) : xch_bytes(XCH_MAX_GROUPS);
+constexpr int64_t SCRATCH_FED_TILES = 128;
+constexpr int64_t SCRATCH_XCH_BYTES = fed_bytes(SCRATCH_FED_TILES) > xch_bytes(XCH_MAX_GROUPS) ? fed_bytes(SCRATCH_FED_TILES) : xch_bytes(XCH_MAX_GROUPS);
 constexpr int64_t SCRATCH_BYTES = SCRATCH_STATE_BYTES + 256 + SCRATCH_XCH_BYTES;
 __device__ __align__(256) uint8_t scratch[SCRATCH_BYTES];
 
@@ -1065,6 +1066,35 @@ int sc_mfma_burn_i8(const int8_t *ops, int32_t iters, int32_t n_groups, int32_t 
     return check_launch("k_mfma_burn");
 }
 
+// A fed launch: heads of 32 rt chunks, and the feeder sets beside them
+// (heads = 0: none).
+struct FedPlan {
+    int32_t rt, heads, sets;
+    int cost;   // per step, DEC_STEP_COST's unit
+};
+constexpr int FED_RT_MAX = 2;
+// Per-step cost of a head's chain at rt = 1, 2, and of ten tiles at their
+// feeders (2,048-token chunks, lossless model).
+constexpr int FED_HEAD_COST[FED_RT_MAX + 1] = {0, 202, 310}, FED_TEN_TILES_COST = 174;
+constexpr int64_t FED_SET_AIM = 6;   // tiles per feeder set while CUs are free
+
+// The cheapest fed launch of n chunks on `cu` CUs with xch_cap bytes of
+// exchange memory: a head's chain or its set's feeders, whichever takes
+// longer, bounds the step.
+static FedPlan fed_plan_of(int64_t n, int64_t cu, int64_t xch_cap, int rt_only) {
+    FedPlan best{};
+    for (int rt = 1; rt <= FED_RT_MAX; ++rt) {
+        const int64_t heads = (n + 32 * rt - 1) / (32 * rt), tiles = heads * rt;
+        if ((rt_only && rt != rt_only) || tiles > FED_MAX_TILES || fed_bytes(tiles) > xch_cap) continue;
+        const int64_t max_sets = (cu - heads) / FED_SLICES;
+        if (max_sets < 1 || (tiles + max_sets - 1) / max_sets > FED_SET_TILES) continue;
+        const int64_t sets = std::min(max_sets, (tiles + FED_SET_AIM - 1) / FED_SET_AIM);
+        const int cost = std::max<int>(FED_HEAD_COST[rt], (int)((tiles + sets - 1) / sets) * FED_TEN_TILES_COST / 10);
+        if (!best.heads || cost < best.cost) best = FedPlan{rt, (int32_t)heads, (int32_t)sets, cost};
+    }
+    return best;
+}
+
 // Workspace of sc_decompress_chunks: the coder state of every chunk between
 // step segments (DecState, 40 bytes each), then the four length statistics
 // of the launch plan, each part 256-byte aligned.
@@ -1075,7 +1105,8 @@ static int64_t dec_state_bytes(int64_t n_chunks) {
 // then the exchange buffers of a fed or split launch
 static int64_t dec_xch_bytes(int64_t n_chunks) {
     const int64_t tiles = (n_chunks + 31) / 32;
-    return std::max(fed_bytes(std::min<int64_t>(tiles, FED_MAX_TILES)), xch_bytes(std::min<int64_t>(tiles, XCH_MAX_GROUPS)));
+    const int64_t fed = (tiles + FED_RT_MAX - 1) / FED_RT_MAX * FED_RT_MAX;   // whole heads
+    return std::max(fed_bytes(std::min<int64_t>(fed, FED_MAX_TILES)), xch_bytes(std::min<int64_t>(tiles, XCH_MAX_GROUPS)));
 }
 // What a call needs at the least (callers that sized their workspace by the
 // split decode's exchange buffers): a launch whose fed exchange does not fit
@@ -1105,16 +1136,6 @@ static void host_len_stats(const int32_t *len, int64_t n, int64_t g0, int64_t G,
         out[1] = std::max(out[1], l1 + at(g0 + G + left - 1 - i) + (l1 > 0 ? 1 : 0));
     }
 }
-
-// A fed launch: workgroups of 32 chunks, and the feeder sets beside them.
-struct FedPlan {
-    int32_t heads, sets;
-};
-constexpr int64_t FED_SET_AIM = 6;   // tiles per feeder set while CUs are free
-
-// Per-step cost of a fed launch, DEC_STEP_COST's unit: a head's chain, or
-// its set's feeders where they take longer (both measured, 2,048-token chunks).
-static int fed_step_cost(const FedPlan &f) { return std::max(222, (f.heads + f.sets - 1) / f.sets * 18); }
 
 // The decode of sc_decompress_chunks with its buffers given: `state` holds
 // DecState for n_chunks rows, `stat_dev` 4 int32 (used only when
@@ -1224,19 +1245,15 @@ static int decompress_run(const sc_model *m, const uint32_t *words, const int64_
     };
     // the fed decode (sc_fed.h) where its heads and feeder sets fit the CUs;
     // SC_HIP_DEC_SPLIT selects the split or unsplit kernels instead
+    const char *fed_env = getenv("SC_HIP_DEC_FED");   // 1 or 2: heads of 32 or 64 chunks (comparisons)
+    const int fed_rt = fed_env ? atoi(fed_env) : 0;
     auto fed_plan = [&](int64_t n) {
-        FedPlan f{};
-        const int64_t tiles = (n + 31) / 32;
-        if (!split_ok || split_force >= 0 || tiles > FED_MAX_TILES || fed_bytes(tiles) > xch_cap) return f;
-        const int64_t max_sets = (cu - tiles) / FED_SLICES;
-        if (max_sets < 1 || (tiles + max_sets - 1) / max_sets > FED_SET_TILES) return f;
-        f.heads = (int32_t)tiles;
-        f.sets = (int32_t)std::min(max_sets, (tiles + FED_SET_AIM - 1) / FED_SET_AIM);
-        return f;
+        if (!split_ok || split_force >= 0 || m->dev.n_layers < FED_MIN_LAYERS) return FedPlan{};
+        return fed_plan_of(n, cu, xch_cap, fed_rt);
     };
     const int p_left = split_p(left);
     const FedPlan f_left = fed_plan(left);
-    const int left_cost = f_left.heads ? fed_step_cost(f_left) : p_left == 8 ? DEC_SPLIT_STEP_COST_P8 : p_left == 4 ? DEC_SPLIT_STEP_COST_P4 : DEC_STEP_COST[1];
+    const int left_cost = f_left.heads ? f_left.cost : p_left == 8 ? DEC_SPLIT_STEP_COST_P8 : p_left == 4 ? DEC_SPLIT_STEP_COST_P4 : DEC_STEP_COST[1];
     const bool pair = can_pair && (int64_t)std::max(0, pair_max - group_max) * DEC_STEP_COST[rt_last] <
                                       (int64_t)left_max * left_cost;
     const int64_t maxlen = std::max(len_max, pair ? pair_max : 0);
@@ -1246,10 +1263,10 @@ static int decompress_run(const sc_model *m, const uint32_t *words, const int64_
         const int64_t rest_last = units == 0 ? n_chunks : pair ? 0 : left;
         const int pl = rest_last ? split_p(rest_last) : 0;
         const FedPlan fl = rest_last ? fed_plan(rest_last) : FedPlan{};
-        std::fprintf(stderr, "sc_decompress_chunks: chunks %lld cu %lld plan [%s] leftover %lld %s steps %lld seg %lld fed %d+%dx%d\n",
+        std::fprintf(stderr, "sc_decompress_chunks: chunks %lld cu %lld plan [%s] leftover %lld %s steps %lld seg %lld fed %d+%dx%d rt %d\n",
                      (long long)n_chunks, (long long)cu, rts.c_str(), (long long)left,
                      left == 0 ? "none" : pair ? "paired" : pl == 8 ? "split launch p8" : pl == 4 ? "split launch p4" : "launch",
-                     (long long)maxlen, (long long)seg, fl.heads, fl.sets, FED_SLICES);
+                     (long long)maxlen, (long long)seg, fl.heads, fl.sets, FED_SLICES, fl.rt);
     }
     int64_t start = 0;
     size_t step = 0;
@@ -1276,12 +1293,14 @@ static int decompress_run(const sc_model *m, const uint32_t *words, const int64_
         int32_t *st = status + start;
         DecState *ds = seg > 0 ? state + start : nullptr;
         if (const FedPlan f = tail ? fed_plan(rest) : FedPlan{}; f.heads) {
-            hipLaunchKernelGGL(k_zero_i32, dim3(16), dim3(256), 0, s, (int32_t *)(xch + f.heads * (int64_t)FED_SUMS),
-                               f.heads * (int64_t)FED_SYNC / 4);
+            const int64_t tiles = (int64_t)f.heads * f.rt;
+            hipLaunchKernelGGL(k_zero_i32, dim3(16), dim3(256), 0, s, (int32_t *)(xch + tiles * FED_SUMS),
+                               tiles * FED_SYNC / 4);
             int rc = check_launch("k_zero_i32");
             if (rc) return rc;
-            const hipError_t e = launch_decompress_fed<1>(m->dev, f.heads, f.sets, s, wds, woff, wcnt, len, count, tokens,
-                                                          toff, st, xch, spin_max);
+            auto *launch = f.rt == 2 ? launch_decompress_fed<2> : launch_decompress_fed<1>;
+            const hipError_t e =
+                launch(m->dev, f.heads, f.sets, s, wds, woff, wcnt, len, count, tokens, toff, st, xch, spin_max);
             if (e == hipSuccess) {
                 rc = check_launch("k_decompress_fed");
                 if (rc) return rc;

@@ -38,8 +38,9 @@ def _decode(codec, monkeypatch, capfd, words, off, cnt, lengths):
 
 
 # heads x sets expected on 256 CUs: one partial tile; a tile and one row; the
-# second set; a tile count that no set count divides; the last size that fits
-@pytest.mark.parametrize("n,heads,sets", [(1, 1, 1), (32, 1, 1), (33, 2, 1), (193, 7, 2), (2049, 65, 11), (4480, 140, 7)])
+# second set; 65 tiles; 64-row heads with a partial last one, and at their limit
+@pytest.mark.parametrize("n,heads,sets", [(1, 1, 1), (32, 1, 1), (33, 2, 1), (193, 7, 2), (2049, 65, 11), (4171, 66, 11),
+                                          (8191, 128, 8)])
 def test_fed_decode_sizes(codec, monkeypatch, capfd, n, heads, sets):
     rng = np.random.default_rng(n)
     lengths = rng.integers(1, 200 if n < 1000 else 90, n)
@@ -54,21 +55,14 @@ def test_fed_decode_sizes(codec, monkeypatch, capfd, n, heads, sets):
     assert shape == (0, 0) and np.array_equal(plain, tokens)
 
 
-def test_fed_decode_beyond_its_limit_runs_unsplit(codec, monkeypatch, capfd):
-    """One chunk more than 140 heads hold: feeders for 141 tiles do not fit."""
-    tokens, lengths, words, off, cnt = _chunks(codec, np.full(4481, 66), 1)
-    back, shape = _decode(codec, monkeypatch, capfd, words, off, cnt, lengths)
-    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
-        assert shape == (0, 0)
-    assert np.array_equal(back, tokens)
-
-
+@pytest.mark.parametrize("rt", ["1", "2"])
 @pytest.mark.parametrize("longest", [1, 2, 3, 63, 64, 65, 129])
-def test_fed_decode_step_edges(codec, monkeypatch, capfd, longest):
+def test_fed_decode_step_edges(codec, monkeypatch, capfd, longest, rt):
     """Few steps (a feeder waits for tokens from the third on) and the
     64-step flush and refill; empty chunks and whole tiles that end early."""
     lengths = np.concatenate([np.full(32, longest), np.zeros(33, int), np.full(40, min(longest, 2)), [longest, 0, 1]])
     tokens, lengths, words, off, cnt = _chunks(codec, lengths, longest)
+    monkeypatch.setenv("SC_HIP_DEC_FED", rt)
     back, shape = _decode(codec, monkeypatch, capfd, words, off, cnt, lengths)
     assert shape[0] > 0 and np.array_equal(back, tokens)
 
