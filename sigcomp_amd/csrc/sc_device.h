@@ -854,13 +854,21 @@ struct EncState {
     int32_t pos;
 };
 
+// a * b for a < 2**40, b < 2**24 (a coder scale times a frequency or a
+// cumulative frequency): the high word of a times b fits the 24-bit multiply
+__device__ __forceinline__ uint64_t mul_scale(uint64_t a, uint32_t b) {
+    const uint64_t low = (uint64_t)(uint32_t)a * b;
+    const uint32_t high = (uint32_t)(low >> 32) + __umul24((uint32_t)(a >> 32), b);
+    return ((uint64_t)high << 32) | (uint32_t)low;
+}
+
 // _encode_one (cpu_entropy_coding.py:121-161) after the frequency lookup.
 // Returns 0 or 1 (capacity exceeded; state left as before the step).
-__device__ __forceinline__ int enc_step(EncState &s, uint64_t cum, uint64_t freq,
+__device__ __forceinline__ int enc_step(EncState &s, uint32_t cum, uint32_t freq,
                                         uint32_t *__restrict__ out, int32_t cap) {
     const uint64_t scale = s.range >> 24;
-    const uint64_t new_range = scale * freq;
-    const uint64_t new_lower = s.lower + scale * cum;
+    const uint64_t new_range = mul_scale(scale, freq);
+    const uint64_t new_lower = s.lower + mul_scale(scale, cum);
     int32_t pos = s.pos, inv = s.inverted;
     if (inv > 0 && new_lower + new_range > new_lower) {
         uint32_t emit_first, emit_rest;
@@ -917,12 +925,6 @@ __device__ __forceinline__ int enc_seal(EncState &s, uint32_t *__restrict__ out,
     s.inverted = 0;
     s.range = ~0ull;
     return 0;
-}
-
-// a * b for a < 2**40, b < 2**24 (a coder scale times a frequency or a
-// cumulative frequency): the high word of a times b fits the 24-bit multiply
-__device__ __forceinline__ uint64_t mul_scale(uint64_t a, uint32_t b) {
-    return (uint64_t)(uint32_t)a * b + ((uint64_t)__umul24((uint32_t)(a >> 32), b) << 32);
 }
 
 // Decoder quantile (point - lower) // scale for 0 < scale < 2**40 (range >>
