@@ -47,13 +47,18 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 constexpr int PAR_DWORDS = 104;
 constexpr int PAR_LDS_DWORDS = 4 * PAR_DWORDS * 4;   // 4 waves x up to 4 n-tiles
 
+// LayerDev::fast of a generic-path layer whose every m0 < 2**31 and shift >=
+// 32 (its stored shifts are whole)
+constexpr int LAYER_FAST_GENERIC = 2;
+
 struct LayerDev {
     const v4i *w;            // packed weight fragments (pack order: pack_weight in sc_kernels.hip)
     const uint32_t *par;     // [n/32][PAR_DWORDS] requant parameter blocks
     int32_t n, kt;           // output width, k-tiles of 32
     int32_t relu;
     int32_t bytes;           // size of the packed weight buffer
-    int32_t fast;            // every m0 < 2**31 and shift >= 32; shift[] holds shift - 32
+    int32_t fast;            // 1: every m0 < 2**31 and shift >= 32; shift[] holds shift - 32
+                             // (CORE_GENERIC: LAYER_FAST_GENERIC, the shifts whole)
     int32_t uni;             // fast, and one m0 and shift for every output (per-tensor constants):
     int32_t um0, ush;        //   that m0 and shift - 32
     int32_t uhi;             //   the pre-shift clamp bounds min(128 * 2**ush - 1, 2**31 - 1)

@@ -23,6 +23,7 @@
 #include <algorithm>
 #include <string>
 
+#include "sc_fed.h"
 #include "sc_gen.h"
 
 namespace sc {
@@ -228,6 +229,337 @@ __global__ __launch_bounds__(256) void k_gen_dec_status(const DecState *__restri
     if (c < n) status[c] = st[c].stat;
 }
 
+// ---- the whole MLP of 32 rows in one workgroup ------------------------------
+//
+// Models whose activations fit the LDS (gen_fused_lds below: every width of
+// a layer up to about 1,500, an embedding width that is a multiple of 16)
+// run fused: a workgroup keeps 32 rows on chip from the token windows to the
+// logits, streams each layer's weights once per 32 rows, and ends with what
+// the call wants of the logits.  The decoder loops over its steps inside
+// one launch.  One launch per stage cost seven launches a step (57 us for 64
+// chunks of a 32 x 64 -> 256 -> 256 x 3 -> 256 model, of which 5 x 6.7 us the
+// layers) and read every operand of every MFMA from memory.  Bound now by
+// the CU's vector L1 (64 B/clock of weights).
+
+enum GenOut { GEN_LOGITS = 0, GEN_CDF = 1, GEN_PAIRS = 2, GEN_DECODE = 3 };
+
+constexpr int GEN_LDS = 156 * 1024;
+constexpr int GEN_BLK = 8;          // k-tiles per block of a layer's loop
+constexpr int GEN_MAX_WINDOW = 256;
+
+// LDS of a fused workgroup, byte offsets (all multiples of 16)
+struct GenLds {
+    int32_t emb, emb_stride, ctx, slots, act[2], ld, logits, dec, bytes;
+    uint32_t inv;   // ceil(2**20 / (emb_dim / 16)): 16-column chunk -> window position
+};
+
+// The rows' coder arrays of GEN_DECODE, after the common part
+struct GenDecLds {
+    static constexpr int SLOT = 0;
+    static constexpr int LOWER = SLOT + WAVES * 2 * 4 * SLOT_DWORDS * 4;
+    static constexpr int RANGE = LOWER + 32 * 8, POINT = RANGE + 32 * 8, WOFF = POINT + 32 * 8, TOFF = WOFF + 32 * 8;
+    static constexpr int RPOS = TOFF + 32 * 8, WCNT = RPOS + 32 * 4, LEN = WCNT + 32 * 4, STAT = LEN + 32 * 4;
+    static constexpr int WBASE = STAT + 32 * 4, WBUF_OFF = WBASE + 32 * 4, RING = WBUF_OFF + 32 * WBUF * 4;
+    static constexpr int LAST = RING + 32 * WIN, MISC = LAST + 32 * 2, BYTES = MISC + 16;
+};
+
+struct GenArgs {
+    const int64_t *ctx;            // GEN_LOGITS, GEN_CDF
+    int8_t *logits;
+    int32_t *cdf, *status;         // status: [1], or [n] in GEN_DECODE
+    const uint8_t *tokens_in;      // GEN_PAIRS
+    const int4 *desc;
+    const int32_t *tile_count;
+    uint2 *pairs;
+    const uint32_t *words;         // GEN_DECODE
+    const int64_t *word_off, *tok_off;
+    const int32_t *word_cnt, *lengths;
+    uint8_t *tokens;
+    int64_t rows;                  // windows, tile descriptors (GEN_PAIRS) or chunks (GEN_DECODE)
+};
+
+// One layer for the workgroup's 32 rows: wave w computes n-tiles w, w + 4,
+// ... two at a time (they share the operand fragments), GEN_BLK k-tiles per
+// block with the next block's weights in flight.  `prep(kt0)` starts block
+// kt0's operand reads, `frag(s)` is its fragment of k-tile kt0 + s.
+template <class PrepFn, class FragFn>
+__device__ __forceinline__ void gen_layer(const LayerDev &L, PrepFn prep, FragFn frag, uint8_t *out, int out_stride,
+                                          int wave, int lane) {
+    const int NT = (L.n + 31) / 32, KT = L.kt, g = lane >> 5, rl = lane & 31, voff = lane * 16;
+    const int lo = L.relu ? 0 : -128;
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)L.w, (short)0, L.bytes, 0x00020000);
+    for (int nt = wave; nt < NT; nt += 2 * WAVES) {
+        const bool two = nt + WAVES < NT;
+        const int nb[2] = {nt, two ? nt + WAVES : nt};
+        v4i w[2][GEN_BLK][2];
+        auto load = [&](int kt0, v4i (&x)[GEN_BLK][2]) __attribute__((always_inline)) {
+            // (past the layer's end: the buffer's bound or the next n-tile's
+            // weights, which are not used)
+#pragma unroll
+            for (int s = 0; s < GEN_BLK; ++s)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) x[s][j] = wload_s(rs, voff, (nb[j] * KT + kt0 + s) * 1024);
+        };
+        v16i acc[2] = {v16i{}, v16i{}};
+        auto block = [&](int kt0, v4i (&cur)[GEN_BLK][2], v4i (&nxt)[GEN_BLK][2]) __attribute__((always_inline)) {
+            if (kt0 + GEN_BLK < KT) load(kt0 + GEN_BLK, nxt);
+            v4i b[GEN_BLK];
+#pragma unroll
+            for (int s = 0; s < GEN_BLK; ++s) b[s] = frag(kt0, s);
+            if (kt0 + GEN_BLK < KT) prep(kt0 + GEN_BLK);
+#pragma unroll
+            for (int s = 0; s < GEN_BLK; ++s)
+                if (kt0 + s < KT) {
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+                        acc[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(cur[s][j], b[s], acc[j], 0, 0, 0);
+                }
+        };
+        prep(0);
+        load(0, w[0]);
+        // the requantisation's parameters behind the first weights
+        v4i pb[2][4], pm[2][4];
+        uint32_t ps[2][4];
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {   // register 4 q + e: feature 8 q + 4 g + e
+                const uint32_t *par = L.par + (int64_t)nb[j] * PAR_DWORDS + 8 * q + 4 * g;
+                pb[j][q] = *(const v4i *)par;
+                pm[j][q] = *(const v4i *)(par + 32);
+                ps[j][q] = L.par[(int64_t)nb[j] * PAR_DWORDS + 64 + 2 * q + g];
+            }
+#pragma unroll 1
+        for (int kt0 = 0; kt0 < KT; kt0 += 2 * GEN_BLK) {
+            block(kt0, w[0], w[1]);
+            if (kt0 + GEN_BLK < KT) block(kt0 + GEN_BLK, w[1], w[0]);
+        }
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            if (j == 1 && !two) break;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int nl = 8 * q + 4 * g;
+                uint32_t pk = 0;
+                // 32-bit high products where the whole layer allows them
+                if (L.fast == LAYER_FAST_GENERIC) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        pk |= requant_u8_fast(acc[j][4 * q + e], pb[j][q][e], pm[j][q][e],
+                                              ((ps[j][q] >> (8 * e)) & 0xFFu) - 32u, lo)
+                              << (8 * e);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        pk |= requant_u8(acc[j][4 * q + e], pb[j][q][e], (uint32_t)pm[j][q][e], (ps[j][q] >> (8 * e)) & 0xFFu, lo)
+                              << (8 * e);
+                }
+                *(uint32_t *)(out + rl * out_stride + nb[j] * 32 + nl) = pk;
+            }
+        }
+    }
+    __syncthreads();
+}
+
+// The MLP: layer 0's operands gathered from the embedding table in LDS by the
+// tokens of slot((position)), the others from the activation buffers; logits
+// at P.logits, PACT_ROW bytes per row.
+template <class SlotFn>
+__device__ __forceinline__ void gen_mlp_rows(const ModelDev &M, const GenLds &P, uint8_t *s_mem, SlotFn slot, int wave,
+                                             int lane) {
+    const int g = lane >> 5, rl = lane & 31, E = M.emb_dim, W = M.window;
+    const uint8_t *s_emb = s_mem + P.emb;
+    const uint16_t *s_ctx = (const uint16_t *)(s_mem + P.ctx);
+    for (int l = 0; l < M.n_layers; ++l) {
+        const LayerDev &L = M.layer[l];
+        const bool last = l == M.n_layers - 1;
+        uint8_t *out = s_mem + (last ? P.logits : P.act[l & 1]);
+        const int stride = last ? PACT_ROW : P.ld;
+        if (l == 0) {
+            int addr[GEN_BLK];
+            gen_layer(
+                L,
+                [&](int kt0) __attribute__((always_inline)) {
+#pragma unroll
+                    for (int s = 0; s < GEN_BLK; ++s) {
+                        // 16 columns of one position (E is a multiple of 16);
+                        // columns past the window have zero weights
+                        // (exact: fewer than 2**12 chunks, 2**20 > 2**12 * chunks per position)
+                        const int ch = (kt0 + s) * 2 + g, p = min((int)(((uint32_t)ch * P.inv) >> 20), W - 1);
+                        addr[s] = (int)s_ctx[slot(p) * 32 + rl] * P.emb_stride + min(ch * 16 - p * E, E - 16);
+                    }
+                },
+                [&](int, int s) __attribute__((always_inline)) { return *(const v4i *)(s_emb + addr[s]); }, out, stride,
+                wave, lane);
+        } else {
+            const uint8_t *in = s_mem + P.act[(l - 1) & 1] + rl * P.ld + 16 * g;
+            gen_layer(
+                L, [](int) {},
+                [&](int kt0, int s) __attribute__((always_inline)) {
+                    return *(const v4i *)(in + min(kt0 + s, L.kt - 1) * 32);
+                },
+                out, stride, wave, lane);
+        }
+    }
+}
+
+template <int OUT>
+__global__ __launch_bounds__(THREADS, 1) void k_gen_fused(ModelDev M, GenLds P, GenArgs A) {
+    __shared__ __attribute__((aligned(16))) uint8_t s_mem[GEN_LDS];
+    __shared__ double s_lut[VOCAB];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int u = lane & 15, q4 = lane >> 4, W = M.window, E = M.emb_dim;
+    uint16_t *s_ctx = (uint16_t *)(s_mem + P.ctx);   // [slot][row]
+    const uint8_t *s_log = s_mem + P.logits;
+    for (int i = threadIdx.x; i < EMB_ROWS * (E / 16); i += THREADS) {
+        const int tok = i / (E / 16), ch = i % (E / 16);
+        *(v4i *)(s_mem + P.emb + tok * P.emb_stride + ch * 16) = *(const v4i *)(M.emb + tok * E + ch * 16);
+    }
+    load_lut_lds(M.lut, s_lut);
+    if constexpr (OUT != GEN_DECODE) {
+        const int64_t tiles = OUT == GEN_PAIRS ? min<int64_t>(*A.tile_count, A.rows) * (R_GEN_TILE / 32) : (A.rows + 31) / 32;
+        for (int64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+            const int64_t r0 = tile * 32;
+            int4 d{};
+            int64_t base = 0;
+            int i0 = 0, valid = 32;
+            if constexpr (OUT == GEN_PAIRS) {
+                d = A.desc[tile / (R_GEN_TILE / 32)];
+                base = (int64_t)(uint32_t)d.x | ((int64_t)d.y << 32);
+                i0 = (int)(tile % (R_GEN_TILE / 32)) * 32;
+                valid = min(32, d.z - i0);
+                if (valid <= 0) continue;   // (the whole workgroup)
+            } else {
+                valid = (int)min<int64_t>(32, A.rows - r0);
+            }
+            __syncthreads();
+            for (int i = threadIdx.x; i < 32 * W; i += THREADS) {
+                const int r = i / W, p = i % W;
+                int tok = SOS;
+                if constexpr (OUT == GEN_PAIRS) {
+                    const int64_t at = (int64_t)i0 + r - W + p;   // step relative to the tile's first
+                    if (r < valid && d.w + at >= 0) tok = A.tokens_in[base + at];
+                } else if (r < valid) {
+                    const int64_t v = A.ctx[(r0 + r) * W + p];
+                    const bool ok = (uint64_t)v <= (uint64_t)SOS;
+                    if (!ok) A.status[0] = SC_STATUS_BAD_TOKEN;
+                    tok = ok ? (int)v : 0;
+                }
+                s_ctx[p * 32 + r] = (uint16_t)tok;
+            }
+            __syncthreads();
+            gen_mlp_rows(M, P, s_mem, [](int p) { return p; }, wave, lane);
+            if constexpr (OUT == GEN_LOGITS) {
+                for (int i = threadIdx.x; i < 32 * 16; i += THREADS) {
+                    const int r = i >> 4, ch = i & 15;
+                    if (r < valid) *(v4i *)(A.logits + (r0 + r) * VOCAB + ch * 16) = *(const v4i *)(s_log + pact_off(r, ch));
+                }
+            } else {
+                for (int gi = wave; gi * 4 < valid; gi += WAVES) {
+                    const int r = gi * 4 + q4;
+                    Freq16 fr;
+                    row_frequencies16(*(const v4i *)(s_log + pact_off(r, u)), s_lut, u, fr);
+                    if (r >= valid) continue;
+                    if constexpr (OUT == GEN_CDF) {
+                        int32_t *dst = A.cdf + (r0 + r) * (VOCAB + 1) + 16 * u;
+                        uint32_t c = fr.ex;
+#pragma unroll
+                        for (int k = 0; k < 16; ++k) {
+                            dst[k] = (int32_t)c;
+                            c += fr.f[k];
+                        }
+                        if (u == 15) dst[16] = (int32_t)TOTAL;
+                    } else {
+                        const int sym = A.tokens_in[base + i0 + r];
+                        if ((sym >> 4) == u) {
+                            uint32_t cum, freq;
+                            freq16_at(fr, sym & 15, cum, freq);
+                            A.pairs[base + i0 + r] = make_uint2(cum, freq);
+                        }
+                    }
+                }
+            }
+        }
+    } else {
+        using D = GenDecLds;
+        uint8_t *dec = s_mem + P.dec;
+        int32_t *s_steps = (int32_t *)(dec + D::MISC);
+        const FedRows c{s_log,
+                        s_lut,
+                        (uint64_t *)(dec + D::LOWER),
+                        (uint64_t *)(dec + D::RANGE),
+                        (uint64_t *)(dec + D::POINT),
+                        (int64_t *)(dec + D::WOFF),
+                        (int64_t *)(dec + D::TOFF),
+                        (int32_t *)(dec + D::RPOS),
+                        (int32_t *)(dec + D::WCNT),
+                        (int32_t *)(dec + D::LEN),
+                        (int32_t *)(dec + D::STAT),
+                        (int32_t *)(dec + D::WBASE),
+                        (uint32_t *)(dec + D::WBUF_OFF),
+                        dec + D::RING,
+                        (uint16_t *)(dec + D::LAST)};
+        uint32_t *slots = (uint32_t *)(dec + D::SLOT) + wave * (2 * 4 * SLOT_DWORDS);
+        const int64_t c0 = (int64_t)blockIdx.x * 32;
+        if (threadIdx.x == 0) *s_steps = 0;
+        for (int i = threadIdx.x; i < 32 * P.slots; i += THREADS) s_ctx[i] = SOS;
+        __syncthreads();
+        if (threadIdx.x < 32) {
+            const int r = threadIdx.x;
+            const int64_t ch = c0 + r;
+            const bool in = ch < A.rows;
+            const int32_t len = in ? A.lengths[ch] : 0, cnt = in ? A.word_cnt[ch] : 0;
+            const int64_t woff = in ? A.word_off[ch] : 0;
+            int take;
+            c.point[r] = dec_init_point(A.words + woff, cnt, take);
+            c.lower[r] = 0ull;
+            c.range[r] = ~0ull;
+            c.rpos[r] = take;
+            c.stat[r] = 0;
+            c.wcnt[r] = cnt;
+            c.woff[r] = woff;
+            c.toff[r] = in ? A.tok_off[ch] : 0;
+            c.len[r] = len;
+            atomicMax(s_steps, len);
+        }
+        for (int i = threadIdx.x; i < 32 * WIN / 4; i += THREADS) ((uint32_t *)c.ring)[i] = 0;
+        __syncthreads();
+        const int32_t steps = *s_steps;
+        auto refill = [&] {   // the next 64 words of every row
+            for (int r = wave; r < 32; r += WAVES) {
+                const int32_t at = c.rpos[r], cnt = c.wcnt[r];
+                c.wbuf[r * WBUF + lane] = at + lane < cnt ? A.words[c.woff[r] + at + lane] : 0u;
+                if (lane == 0) c.wbase[r] = at;
+            }
+        };
+        refill();
+        __syncthreads();
+        const int mask = P.slots - 1;   // the window's ring has a power of two slots
+#pragma unroll 1
+        for (int32_t t = 0; t < steps; ++t) {
+            gen_mlp_rows(M, P, s_mem, [&](int p) { return (t - W + p) & mask; }, wave, lane);
+            for (int gi = wave; gi < 8; gi += 2 * WAVES) {
+                const int ra = gi * 4 + q4, rb = ra + 4 * WAVES;
+                const bool a = __builtin_amdgcn_ballot_w64(t < c.len[ra] && c.stat[ra] == 0) != 0;
+                const bool b = __builtin_amdgcn_ballot_w64(t < c.len[rb] && c.stat[rb] == 0) != 0;
+                if (a && b) fed_decode_rows<2>(c, slots, t, gi, lane);
+                else if (a) fed_decode_rows<1>(c, slots, t, gi, lane);
+                else if (b) fed_decode_rows<1>(c, slots, t, gi + WAVES, lane);
+            }
+            __syncthreads();
+            if (threadIdx.x < 32) s_ctx[(t & mask) * 32 + threadIdx.x] = c.ring[threadIdx.x * WIN + (t & (WIN - 1))];
+            if ((t & (WIN - 1)) == WIN - 1 || t == steps - 1) {
+                const int32_t p = (t & ~(WIN - 1)) + lane;
+                for (int r = wave; r < 32; r += WAVES)
+                    if (p <= t && p < c.len[r]) A.tokens[c.toff[r] + p] = c.ring[r * WIN + lane];
+                refill();
+            }
+            __syncthreads();
+        }
+        if (threadIdx.x < 32 && c0 + threadIdx.x < A.rows) A.status[c0 + threadIdx.x] = c.stat[threadIdx.x];
+    }
+}
+
 // ---- logits -> int32 CDF (sc_mlp_forward_cdf) ------------------------------
 
 __global__ __launch_bounds__(256) void k_gen_cdf32(const int8_t *__restrict__ logits, int64_t rows,
@@ -255,6 +587,41 @@ __global__ __launch_bounds__(256) void k_gen_cdf32(const int8_t *__restrict__ lo
 
 int64_t round_up(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
 
+// The fused kernel's LDS for a model; bytes = 0 when it does not fit.
+GenLds gen_fused_lds(const ModelDev &M) {
+    GenLds P{};
+    if (M.emb_dim % 16 || M.window > GEN_MAX_WINDOW) return P;
+    P.slots = 1;
+    while (P.slots < M.window) P.slots *= 2;
+    int64_t ld = 0;   // activation rows: the widest hidden layer and a 16-byte pad (bank spread)
+    for (int i = 0; i + 1 < M.n_layers; ++i) ld = std::max<int64_t>(ld, round_up(M.layer[i].n, 32) + 16);
+    P.emb_stride = M.emb_dim + 16;
+    P.inv = ((1u << 20) + M.emb_dim / 16 - 1) / (M.emb_dim / 16);
+    int64_t at = 0;
+    auto take = [&](int64_t bytes) {
+        const int64_t o = at;
+        at += round_up(bytes, 16);
+        return o;
+    };
+    P.emb = (int32_t)take((int64_t)EMB_ROWS * P.emb_stride);
+    P.ctx = (int32_t)take((int64_t)P.slots * 64);
+    P.ld = (int32_t)std::min<int64_t>(ld, GEN_LDS);
+    P.act[0] = (int32_t)take(32 * (int64_t)P.ld);
+    P.act[1] = (int32_t)take(32 * (int64_t)P.ld);
+    P.logits = (int32_t)take(32 * PACT_ROW);
+    P.dec = (int32_t)take(GenDecLds::BYTES);
+    P.bytes = at <= GEN_LDS && ld <= GEN_LDS ? (int32_t)at : 0;
+    return P;
+}
+
+// Workgroups of a fused launch over `tiles` 32-row tiles: one per CU.
+unsigned fused_grid(int64_t tiles) {
+    int dev = 0, cu = 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+        cu = 256;
+    return (unsigned)std::max<int64_t>(1, std::min<int64_t>(tiles, cu));
+}
+
 // Widest padded layer input / output of the model (bytes per row).
 int64_t max_width(const ModelDev &M) {
     int64_t w = round_up((int64_t)M.window * M.emb_dim, 32);
@@ -275,6 +642,13 @@ int64_t batch_rows(const ModelDev &M, int64_t needed, int64_t unit) {
 }
 
 hipError_t launch_check() { return hipGetLastError(); }
+
+int fused_result(const char *what, std::string &err) {
+    const hipError_t e = launch_check();
+    if (e == hipSuccess) return SC_OK;
+    err = std::string(what) + hipGetErrorString(e);
+    return SC_ERR_HIP;
+}
 
 // Stream-ordered scratch of one call (hipMallocAsync / hipFreeAsync).
 struct Scratch {
@@ -319,6 +693,17 @@ hipError_t gen_mlp(const ModelDev &M, const GenRows &g, int64_t rows, int8_t *X0
 
 int gen_mlp_forward(const ModelDev &M, const int64_t *ctx, int64_t rows, int8_t *logits, int32_t *cdf,
                     int32_t *status, hipStream_t s, std::string &err) {
+    if (const GenLds P = gen_fused_lds(M); P.bytes) {
+        GenArgs A{};
+        A.ctx = ctx;
+        A.logits = logits;
+        A.cdf = cdf;
+        A.status = status;
+        A.rows = rows;
+        hipLaunchKernelGGL(cdf ? k_gen_fused<GEN_CDF> : k_gen_fused<GEN_LOGITS>, dim3(fused_grid((rows + 31) / 32)),
+                           dim3(THREADS), 0, s, M, P, A);
+        return fused_result("generic MLP launch: ", err);
+    }
     const int64_t B = batch_rows(M, rows, 64);
     const int64_t width = max_width(M), rows_p = B;
     Scratch scr(s);
@@ -348,6 +733,17 @@ int gen_mlp_forward(const ModelDev &M, const int64_t *ctx, int64_t rows, int8_t 
 
 int gen_compress(const ModelDev &M, const uint8_t *tokens, const int32_t *tile_start, int64_t n_chunks,
                  const int4 *desc, int64_t max_tiles, uint2 *pairs, hipStream_t s, std::string &err) {
+    if (const GenLds P = gen_fused_lds(M); P.bytes) {
+        GenArgs A{};
+        A.tokens_in = tokens;
+        A.desc = desc;
+        A.tile_count = tile_start + n_chunks;
+        A.pairs = pairs;
+        A.rows = max_tiles;
+        hipLaunchKernelGGL(k_gen_fused<GEN_PAIRS>, dim3(fused_grid(max_tiles * (R_GEN_TILE / 32))), dim3(THREADS), 0, s, M,
+                           P, A);
+        return fused_result("generic compress launch: ", err);
+    }
     const int64_t rows_b = batch_rows(M, max_tiles * R_GEN_TILE, R_GEN_TILE), width = max_width(M);
     const int64_t tiles_per = rows_b / R_GEN_TILE;
     Scratch scr(s);
@@ -376,6 +772,19 @@ int gen_compress(const ModelDev &M, const uint8_t *tokens, const int32_t *tile_s
 int gen_decompress(const ModelDev &M, const uint32_t *words, const int64_t *word_off, const int32_t *word_cnt,
                    const int32_t *lengths, int64_t n_chunks, uint8_t *tokens, const int64_t *tok_off,
                    int32_t *status, DecState *state, int32_t max_len, hipStream_t s, std::string &err) {
+    if (const GenLds P = gen_fused_lds(M); P.bytes) {
+        GenArgs A{};
+        A.status = status;
+        A.words = words;
+        A.word_off = word_off;
+        A.word_cnt = word_cnt;
+        A.lengths = lengths;
+        A.tokens = tokens;
+        A.tok_off = tok_off;
+        A.rows = n_chunks;
+        hipLaunchKernelGGL(k_gen_fused<GEN_DECODE>, dim3((unsigned)((n_chunks + 31) / 32)), dim3(THREADS), 0, s, M, P, A);
+        return fused_result("generic decompress launch: ", err);
+    }
     const int64_t width = max_width(M);
     const int64_t B = batch_rows(M, n_chunks, 64), rows_p = B;
     Scratch scr(s);

@@ -895,10 +895,11 @@ int sc_model_create(const int8_t *emb, int32_t emb_rows, int32_t emb_dim, int32_
             sh[j] = (uint8_t)sj;
             fast = fast && mj < (int64_t(1) << 31) && sj >= 32;
         }
-        fast = fast && special;   // the generic path requantises with the full 64-bit form
+        const bool fast_generic = fast && !special;
+        fast = fast && special;
         if (fast)
             for (int j = 0; j < L.n; ++j) sh[j] = (uint8_t)(sh[j] - 32);
-        D.fast = fast ? 1 : 0;
+        D.fast = fast ? 1 : fast_generic ? LAYER_FAST_GENERIC : 0;
         // per-tensor constants: one m0 and shift for the whole layer
         bool uni = fast;
         for (int j = 1; j < L.n && uni; ++j) uni = m0[j] == m0[0] && sh[j] == sh[0];

@@ -1,0 +1,52 @@
+"""GPU tests of the fused generic kernel: architectures at the edges of what
+it takes (embedding widths that are multiples of 16, windows that are no
+power of two, widths that are no multiple of 32, one and many layers) and
+just beyond it, against the oracle."""
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+# window, embedding width, hidden width, hidden layers: an odd k-tile count
+# with a half tile of padding; more n-tiles than two per wave; a deep, narrow
+# one; a window of 65; just too wide for the LDS (separate launches)
+ARCHS = {"half_tile": (3, 16, 80, 2), "wide": (16, 32, 608, 1), "deep": (7, 48, 32, 12), "window65": (65, 16, 96, 2),
+         "one_layer": (33, 64, 0, 0), "beyond": (4, 32, 2080, 1)}
+
+
+@pytest.fixture(scope="module", params=sorted(ARCHS))
+def arch(request):
+    if not torch.cuda.is_available():
+        pytest.fail("GPU tests need a HIP device")
+    from sigcomp_amd.model_io import random_int_model
+    from sigcomp_amd.quant_mlp_export import QuantMLPCompression
+    w, e, h, nh = ARCHS[request.param]
+    m = random_int_model(seed=3 + nh, window=w, emb_dim=e, hidden=max(h, 1), n_hidden=nh, per_channel=True)
+    return m, QuantMLPCompression(chunk_len=300, gpu=0, model=m)
+
+
+@pytest.mark.parametrize("rows", [1, 31, 33, 100])
+def test_forward(arch, oracle_mod, rows):
+    m, codec = arch
+    ctx = np.random.default_rng(rows).integers(0, 257, (rows, m.window)).astype(np.int64)
+    ref = oracle_mod.mlp_forward(oracle_mod.OracleModel(m), ctx)
+    dev = torch.from_numpy(ctx).cuda()
+    assert np.array_equal(codec.hip.forward_windows(dev, "logits").cpu().numpy(), ref)
+    cdf = codec.hip.forward_windows(dev, "cdf").cpu().numpy().astype(np.int64)
+    assert np.array_equal(cdf, oracle_mod.logits_to_cdf(ref, m.exp_lut))
+
+
+def test_round_trip_and_corrupt_chunk(arch, oracle_mod):
+    m, codec = arch
+    rng = np.random.default_rng(8)
+    lengths = [1, 2, 31, 63, 64, 65, 127, 129, 0, 200] + list(rng.integers(1, 70, 30))
+    chunks = [rng.integers(0, 60, n).astype(np.uint8) for n in lengths]
+    enc = codec.compress_chunks(chunks)
+    assert enc == oracle_mod.compress_chunks(oracle_mod.OracleModel(m), chunks)
+    assert all(np.array_equal(a, b) for a, b in zip(chunks, codec.decompress_chunks(enc, lengths)))
+    enc[4] = b"\xff" * 8
+    with pytest.raises(ValueError, match="chunk 4"):
+        codec.decompress_chunks(enc, lengths)
