@@ -53,7 +53,7 @@ constexpr int64_t fed_bytes(int64_t tiles) { return tiles * (FED_SUMS + FED_SYNC
 
 // Host launchers (stream-ordered, no error check: the caller checks
 // hipGetLastError).  The MLP core follows M.pipe.
-template <int MODE>
+template <int MODE, int RT>
 void launch_mlp_context(const ModelDev &M, unsigned grid, hipStream_t s, const int64_t *ctx, int64_t rows,
                         int8_t *logits, int32_t *cdf, int32_t *status);
 void launch_compress_mlp(const ModelDev &M, unsigned grid, hipStream_t s, const uint8_t *tokens, int64_t n_chunks,
@@ -113,19 +113,20 @@ constexpr int act_row_bytes() { return PIPE ? PACT_ROW : ACT_ROW; }
 template <bool PIPE>
 __device__ __forceinline__ int act_at(int r, int chunk) { return PIPE ? pact_off(r, chunk) : act_off(r, chunk); }
 
-template <int MODE, int CORE>
+template <int MODE, int CORE, int RT>
 __global__ __launch_bounds__(THREADS, 1) void k_mlp_context(ModelDev M, const int64_t *__restrict__ ctx,
                                                             int64_t rows, int8_t *__restrict__ logits,
                                                             int32_t *__restrict__ cdf,
                                                             int32_t *__restrict__ status) {
     constexpr bool PIPE = CORE != CORE_PLAIN;
+    constexpr int ROWS = 32 * RT;   // per tile
     __shared__ __attribute__((aligned(16))) uint8_t s_emb[EMB_BYTES];
-    __shared__ __attribute__((aligned(16))) uint8_t s_act[R_TILE * act_row_bytes<PIPE>()];
+    __shared__ __attribute__((aligned(16))) uint8_t s_act[ROWS * act_row_bytes<PIPE>()];
     // rows padded to CTX_STRIDE halfwords: layer 0 reads one position of 32
     // consecutive rows at a time, which a 128-byte row stride would put in
     // one LDS bank
     constexpr int CTX_STRIDE = WIN + 2;
-    __shared__ __attribute__((aligned(16))) uint16_t s_ctx[R_TILE * CTX_STRIDE];
+    __shared__ __attribute__((aligned(16))) uint16_t s_ctx[ROWS * CTX_STRIDE];
     __shared__ __attribute__((aligned(16))) uint32_t s_par[par_lds_dwords<CORE>()];
     __shared__ double s_lut[VOCAB];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -133,17 +134,17 @@ __global__ __launch_bounds__(THREADS, 1) void k_mlp_context(ModelDev M, const in
     load_emb_lds(M.emb, s_emb);
     load_lut_lds(M.lut, s_lut);
     mlp_tile_init<CORE>(M, s_par, wave, lane);
-    const int64_t n_tiles = (rows + R_TILE - 1) / R_TILE;
-    // A tile's 128 x 64 context tokens: 32 per thread, all loads issued
+    const int64_t n_tiles = (rows + ROWS - 1) / ROWS;
+    // A tile's context tokens (128 x 64: 32 per thread), all loads issued
     // before the first is used (a load / wait / store loop costs one memory
     // round trip per token).  Element j * THREADS + thread is row 4j + wave,
     // position lane: each load instruction reads 2 KB.  Addresses and row
     // limits are formed from per-tile values, so that none is hoisted out of
     // the tile loop (32 such registers held across the MLP make it spill).
-    constexpr int CTX_PER = R_TILE * WIN / THREADS;
+    constexpr int CTX_PER = ROWS * WIN / THREADS;
     static_assert(THREADS == 4 * WIN, "four context rows per load instruction");
     for (int64_t tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
-        const int64_t row0 = tile * R_TILE;
+        const int64_t row0 = tile * ROWS;
         const int64_t *src = ctx + row0 * WIN + threadIdx.x;
         const int64_t lim = rows - row0 - wave;   // element j is in range iff 4j < lim
         int64_t v[CTX_PER];
@@ -160,18 +161,18 @@ __global__ __launch_bounds__(THREADS, 1) void k_mlp_context(ModelDev M, const in
         }
         if (bad) status[0] = SC_STATUS_BAD_TOKEN;
         __syncthreads();
-        mlp_tile<CORE, RT_TILE>(M, s_emb, s_act, s_par, [&](int r, int p) { return (int)s_ctx[r * CTX_STRIDE + p]; },
+        mlp_tile<CORE, RT>(M, s_emb, s_act, s_par, [&](int r, int p) { return (int)s_ctx[r * CTX_STRIDE + p]; },
                                 wave, lane);
         if (MODE == OUT_LOGITS) {
             // 128 rows x 256 bytes, 16-byte chunks, coalesced
-            for (int i = threadIdx.x; i < R_TILE * 16; i += THREADS) {
+            for (int i = threadIdx.x; i < ROWS * 16; i += THREADS) {
                 const int r = i >> 4, c = i & 15;
                 if (row0 + r < rows)
                     *(v4i *)(logits + (row0 + r) * VOCAB + c * 16) = *(const v4i *)(s_act + act_at<PIPE>(r, c));
             }
         } else {
             // two row groups (gi, gi + WAVES) per iteration, see row_frequencies16n
-            for (int gi = wave; gi < R_TILE / 4; gi += 2 * WAVES) {
+            for (int gi = wave; gi < ROWS / 4; gi += 2 * WAVES) {
                 const int rr[2] = {gi * 4 + q4, (gi + WAVES) * 4 + q4};
                 const v4i raw[2] = {*(const v4i *)(s_act + act_at<PIPE>(rr[0], u)),
                                     *(const v4i *)(s_act + act_at<PIPE>(rr[1], u))};

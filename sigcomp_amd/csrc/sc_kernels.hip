@@ -957,6 +957,25 @@ const uint64_t *sc_model_lut(const sc_model *m) { return m ? m->dev.lut : nullpt
 
 int sc_model_core(const sc_model *m) { return m ? m->dev.pipe : 0; }
 
+// Row tiles per workgroup of an explicit-context launch: a tile's time is
+// the weight stream's at 32 rows and the products' at 128, so rows that one
+// wave of smaller tiles holds finish sooner in them (CTX_TILE_COST: us of one
+// wave of 256 tiles; measured, 32 .. 128-row tiles: 1,000 rows 63, 68, 83, 107
+// us, 16,384 rows 137, 88, 101, 121, 32,768 rows 263, 169, 197, 148).
+static int ctx_row_tiles(int64_t rows, int64_t cu) {
+    constexpr int CTX_TILE_COST[5] = {0, 66, 84, 112, 146};
+    int best = 4;
+    int64_t cost = INT64_MAX;
+    for (int rt = 4; rt >= 1; --rt) {
+        const int64_t tiles = (rows + 32 * rt - 1) / (32 * rt), c = (tiles + cu - 1) / cu * CTX_TILE_COST[rt];
+        if (c < cost) {
+            cost = c;
+            best = rt;
+        }
+    }
+    return best;
+}
+
 static int mlp_context_launch(const sc_model *m, const int64_t *ctx, int64_t rows, int8_t *logits,
                               int32_t *cdf, int32_t *status, void *stream, int mode) {
     if (!m || rows < 0 || !status) return fail(SC_ERR_ARG, "bad argument");
@@ -970,10 +989,22 @@ static int mlp_context_launch(const sc_model *m, const int64_t *ctx, int64_t row
                                        mode == OUT_CDF32 ? cdf : nullptr, status, as_stream(stream), err);
         return rc ? fail(rc, err) : SC_OK;
     }
-    const int64_t tiles = (rows + R_TILE - 1) / R_TILE;
-    const int grid = (int)std::min<int64_t>(tiles, m->n_cu);
-    if (mode == OUT_LOGITS) launch_mlp_context<OUT_LOGITS>(m->dev, grid, as_stream(stream), ctx, rows, logits, cdf, status);
-    else launch_mlp_context<OUT_CDF32>(m->dev, grid, as_stream(stream), ctx, rows, logits, cdf, status);
+    const int rt = ctx_row_tiles(rows, m->n_cu);
+    const int64_t tiles = (rows + 32 * rt - 1) / (32 * rt);
+    const unsigned grid = (unsigned)std::min<int64_t>(tiles, m->n_cu);
+    switch (rt) {
+#define SC_CTX_CASE(N)                                                                                             \
+    case N:                                                                                                        \
+        if (mode == OUT_LOGITS)                                                                                    \
+            launch_mlp_context<OUT_LOGITS, N>(m->dev, grid, as_stream(stream), ctx, rows, logits, cdf, status);    \
+        else launch_mlp_context<OUT_CDF32, N>(m->dev, grid, as_stream(stream), ctx, rows, logits, cdf, status);    \
+        break;
+        SC_CTX_CASE(1)
+        SC_CTX_CASE(2)
+        SC_CTX_CASE(3)
+        SC_CTX_CASE(4)
+#undef SC_CTX_CASE
+    }
     return check_launch("k_mlp_context");
 }
 
