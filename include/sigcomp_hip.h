@@ -122,6 +122,17 @@ int sc_mlp_forward(const sc_model *model, const int64_t *ctx, int64_t rows, int8
 int sc_mlp_forward_cdf(const sc_model *model, const int64_t *ctx, int64_t rows, int32_t *cdf,
                        int32_t *status, void *stream);
 
+/* sc_mlp_forward (logits non-null) or sc_mlp_forward_cdf (cdf non-null;
+ * exactly one of them) with device workspace: with at least
+ * sc_mlp_forward_workspace_bytes(rows) bytes, calls of few rows run in two
+ * launches, layer 0 spread over the device and then the rest (the same
+ * results); with less, and for calls that this does not help (0 bytes), as
+ * without workspace.  Replaces GPUBitExactMLPDecoder._ar_step
+ * (quant_mlp_export.py:133-138) as those do. */
+int64_t sc_mlp_forward_workspace_bytes(int64_t rows);
+int sc_mlp_forward_ws(const sc_model *model, const int64_t *ctx, int64_t rows, int8_t *logits, int32_t *cdf,
+                      int32_t *status, void *workspace, int64_t workspace_bytes, void *stream);
+
 /* int8 logits [rows, 256] + LUT (device uint64/int64 [256]) -> int64 CDF
  * [rows, 257].  Replaces int8_logits_to_cdf (gpu_entropy_coding.py:25-51). */
 int sc_logits_to_cdf(const int8_t *logits, int64_t rows, const uint64_t *lut, int64_t *cdf,

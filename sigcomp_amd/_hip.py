@@ -28,7 +28,7 @@ SC_STATUS_SYNC_TIMEOUT = 4
 EXPORTED = (
     "sc_last_error", "sc_version", "sc_model_create", "sc_model_destroy", "sc_model_lut",
     "sc_model_core",
-    "sc_mlp_forward", "sc_mlp_forward_cdf", "sc_logits_to_cdf", "sc_encode_step",
+    "sc_mlp_forward", "sc_mlp_forward_ws", "sc_mlp_forward_workspace_bytes", "sc_mlp_forward_cdf", "sc_logits_to_cdf", "sc_encode_step",
     "sc_encode_seal", "sc_decode_step", "sc_compress_workspace_bytes", "sc_compress_chunks",
     "sc_decompress_workspace_bytes", "sc_decompress_chunks", "sc_decompress_chunks_opts",
     "sc_decompress_chunks_static",
@@ -89,6 +89,9 @@ def lib():
         L.sc_model_core.argtypes = [_P]
         L.sc_mlp_forward.argtypes = [_P, _P, _I64, _P, _P, _P]
         L.sc_mlp_forward_cdf.argtypes = [_P, _P, _I64, _P, _P, _P]
+        L.sc_mlp_forward_workspace_bytes.argtypes = [_I64]
+        L.sc_mlp_forward_workspace_bytes.restype = _I64
+        L.sc_mlp_forward_ws.argtypes = [_P, _P, _I64, _P, _P, _P, _P, _I64, _P]
         L.sc_logits_to_cdf.argtypes = [_P, _I64, _P, _P, _P]
         L.sc_encode_step.argtypes = [_P, _P, _P, _P, _I64, _I64, ctypes.POINTER(EncoderState), _P,
                                      _I64, _P]

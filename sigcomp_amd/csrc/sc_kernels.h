@@ -56,6 +56,10 @@ constexpr int64_t fed_bytes(int64_t tiles) { return tiles * (FED_SUMS + FED_SYNC
 template <int MODE, int RT>
 void launch_mlp_context(const ModelDev &M, unsigned grid, hipStream_t s, const int64_t *ctx, int64_t rows,
                         int8_t *logits, int32_t *cdf, int32_t *status);
+// The same in two launches (sc_ctx_two.hip, pipelined cores): exactly one of
+// logits and cdf; feat = 512 bytes per row of whole 32-row tiles.
+void launch_ctx_two(const ModelDev &M, hipStream_t s, const int64_t *ctx, int64_t rows, int8_t *logits, int32_t *cdf,
+                    int32_t *status, uint8_t *feat);
 void launch_compress_mlp(const ModelDev &M, unsigned grid, hipStream_t s, const uint8_t *tokens, int64_t n_chunks,
                          const int32_t *tile_start, const int4 *desc, int64_t max_desc, uint2 *pairs);
 template <int RT>

@@ -1018,6 +1018,31 @@ int sc_mlp_forward_cdf(const sc_model *m, const int64_t *ctx, int64_t rows, int3
     return mlp_context_launch(m, ctx, rows, nullptr, cdf, status, stream, OUT_CDF32);
 }
 
+// Rows up to which the two-launch form is used: layer 0's launch grows by a
+// round of 512 workgroups per 1,024 rows, one wave of 32-row tiles of the
+// whole MLP takes the same time for up to 8,192 (62 us; two launches: 25 us
+// at 1 row, 29 at 1,000, 36 at 2,048, 53 at 4,096).
+constexpr int64_t CTX_TWO_MAX_ROWS = 4096;
+
+int64_t sc_mlp_forward_workspace_bytes(int64_t rows) {
+    if (rows < 0) return -1;
+    return rows <= CTX_TWO_MAX_ROWS ? (rows + 31) / 32 * 32 * HID : 0;
+}
+
+int sc_mlp_forward_ws(const sc_model *m, const int64_t *ctx, int64_t rows, int8_t *logits, int32_t *cdf,
+                      int32_t *status, void *workspace, int64_t workspace_bytes, void *stream) {
+    if (!m || rows < 0 || !status) return fail(SC_ERR_ARG, "bad argument");
+    if (rows == 0) return SC_OK;
+    if ((!logits) == (!cdf)) return fail(SC_ERR_ARG, "exactly one of logits and cdf");
+    const int64_t need = sc_mlp_forward_workspace_bytes(rows);
+    if (need == 0 || !workspace || workspace_bytes < need || !ctx ||
+        (m->dev.pipe != CORE_PIPE_UNI && m->dev.pipe != CORE_PIPE))
+        return mlp_context_launch(m, ctx, rows, logits, cdf, status, stream, logits ? OUT_LOGITS : OUT_CDF32);
+    DeviceGuard guard(m->device);
+    launch_ctx_two(m->dev, as_stream(stream), ctx, rows, logits, cdf, status, (uint8_t *)workspace);
+    return check_launch("k_ctx_layer0 / k_ctx_rest");
+}
+
 int sc_logits_to_cdf(const int8_t *logits, int64_t rows, const uint64_t *lut, int64_t *cdf, void *stream) {
     if (rows < 0) return fail(SC_ERR_ARG, "rows must be nonnegative");
     if (rows == 0) return SC_OK;

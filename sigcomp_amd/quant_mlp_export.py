@@ -126,12 +126,13 @@ class HipModel:
         with torch.cuda.device(self.device):
             if out == "logits":
                 res = torch.empty((rows, VOCAB_SIZE), dtype=torch.int8, device=self.device)
-                fn = _hip.lib().sc_mlp_forward
             else:
                 res = torch.empty((rows, VOCAB_SIZE + 1), dtype=torch.int32, device=self.device)
-                fn = _hip.lib().sc_mlp_forward_cdf
-            _hip.check(fn(self.handle, _hip.ptr(ctx), rows, _hip.ptr(res), _hip.ptr(status),
-                          _hip.stream_ptr()))
+            nbytes = int(_hip.lib().sc_mlp_forward_workspace_bytes(rows))
+            ws = torch.empty(nbytes, dtype=torch.uint8, device=self.device) if nbytes else None
+            to = (_hip.ptr(res), None) if out == "logits" else (None, _hip.ptr(res))
+            _hip.check(_hip.lib().sc_mlp_forward_ws(self.handle, _hip.ptr(ctx), rows, *to, _hip.ptr(status),
+                                                    _hip.ptr(ws) if nbytes else None, nbytes, _hip.stream_ptr()))
         if int(status.item()) != 0:
             raise ValueError("context tokens must be in [0, 256]")
         return res

@@ -28,7 +28,7 @@ def codec(request, int_models):
     return m, c
 
 
-@pytest.mark.parametrize("rows", [1, 33, 32 * N_CU, 32 * N_CU + 1, 64 * N_CU + 7, 96 * N_CU + 95])
+@pytest.mark.parametrize("rows", [1, 33, 4096, 4097, 32 * N_CU, 32 * N_CU + 1, 64 * N_CU + 7, 96 * N_CU + 95])
 def test_tile_sizes(codec, oracle_mod, rows):
     m, c = codec
     rng = np.random.default_rng(rows)
@@ -44,3 +44,15 @@ def test_tile_sizes(codec, oracle_mod, rows):
     # every row, through calls of another tile size
     again = np.concatenate([c.hip.forward_windows(dev[i:i + 5000], "logits").cpu().numpy() for i in range(0, rows, 5000)])
     assert np.array_equal(again, logits)
+
+
+def test_no_rows_and_bad_token(codec):
+    _, c = codec
+    empty = torch.zeros((0, 64), dtype=torch.int64, device="cuda")
+    assert c.hip.forward_windows(empty, "logits").shape == (0, 256)
+    assert c.hip.forward_windows(empty, "cdf").shape == (0, 257)
+    for bad in (-1, 257):
+        ctx = torch.zeros((70, 64), dtype=torch.int64, device="cuda")
+        ctx[69, 63] = bad
+        with pytest.raises(ValueError):
+            c.hip.forward_windows(ctx, "logits")
