@@ -52,11 +52,29 @@ def _device_of(t: torch.Tensor) -> torch.device:
     return t.device
 
 
+def _on(t, device, dtype) -> torch.Tensor:
+    """`t` as a contiguous tensor of `dtype` on `device`: itself when it is
+    one (what a step loop passes; the conversions below cost more host time
+    than the step's launch)."""
+    if isinstance(t, torch.Tensor) and t.dtype is dtype and t.device == device and t.is_contiguous():
+        return t
+    return torch.as_tensor(t).to(device, dtype).contiguous()
+
+
 def _lut_on(exp_lut, device) -> torch.Tensor:
-    lut = torch.as_tensor(exp_lut, dtype=torch.int64)
+    lut = _on(exp_lut, device, torch.int64)
     if lut.shape != (VOCAB_SIZE,):
         raise ValueError("exp_lut must have shape (256,)")
-    return lut.to(device).contiguous()
+    return lut
+
+
+def _launch(device, fn, *args) -> None:
+    """fn(*args, stream) on `device`'s current stream."""
+    if torch.cuda.current_device() == device.index:
+        _hip.check(fn(*args, _hip.stream_ptr()))
+    else:
+        with torch.cuda.device(device):
+            _hip.check(fn(*args, _hip.stream_ptr()))
 
 
 def int8_logits_to_cdf(int8_logits, exp_lut, precision=PRECISION):
@@ -95,6 +113,7 @@ class GpuRangeStepEncoder:
         self._state = _hip.EncoderState(
             _hip.ptr(self.state_lower), _hip.ptr(self.state_range), _hip.ptr(self.num_inverted),
             _hip.ptr(self.first_inv_word), _hip.ptr(self.write_pos), _hip.ptr(self.status))
+        self._dev = self.state_lower.device   # with its index
         self._sealed = False
 
     def encode_step_int8(self, int8_logits, exp_lut, symbols, valid_lens_tensor, t):
@@ -104,16 +123,15 @@ class GpuRangeStepEncoder:
             raise ValueError("t must be nonnegative")
         if int8_logits.dtype != torch.int8 or tuple(int8_logits.shape) != (self.B, VOCAB_SIZE):
             raise ValueError("int8_logits must have shape (batch, 256)")
-        logits = int8_logits.to(self.device).contiguous()
-        syms = torch.as_tensor(symbols).to(self.device, torch.int64).contiguous()
-        valid = torch.as_tensor(valid_lens_tensor).to(self.device, torch.int64).contiguous()
+        dev = self._dev
+        logits = _on(int8_logits, dev, torch.int8)
+        syms = _on(symbols, dev, torch.int64)
+        valid = _on(valid_lens_tensor, dev, torch.int64)
         if syms.shape != (self.B,) or valid.shape != (self.B,):
             raise ValueError("symbols and valid_lens must have shape (batch,)")
-        lut = _lut_on(exp_lut, self.device)
-        with torch.cuda.device(self.device):
-            _hip.check(_hip.lib().sc_encode_step(
-                _hip.ptr(logits), _hip.ptr(lut), _hip.ptr(syms), _hip.ptr(valid), int(t), self.B,
-                self._state, _hip.ptr(self.output_words), self.max_words, _hip.stream_ptr()))
+        lut = _lut_on(exp_lut, dev)
+        _launch(dev, _hip.lib().sc_encode_step, _hip.ptr(logits), _hip.ptr(lut), _hip.ptr(syms), _hip.ptr(valid), int(t),
+                self.B, self._state, _hip.ptr(self.output_words), self.max_words)
 
     def seal(self):
         if self._sealed:
@@ -181,6 +199,7 @@ class GpuRangeDecoder:
         self._state = _hip.DecoderState(
             _hip.ptr(self.state_lower), _hip.ptr(self.state_range), _hip.ptr(self.point),
             _hip.ptr(self.read_pos), _hip.ptr(self.end_pos), _hip.ptr(self.status))
+        self._dev = self.state_lower.device   # with its index
 
     def decode_step_int8(self, int8_logits, exp_lut, valid_lens_tensor, t):
         """Decoded symbols of step ``t`` (int64 [B]; 256 for inactive streams).
@@ -191,15 +210,14 @@ class GpuRangeDecoder:
             raise ValueError("int8_logits must have shape (batch, 256)")
         if t < 0:
             raise ValueError("t must be nonnegative")
-        logits = int8_logits.to(self.device).contiguous()
-        valid = torch.as_tensor(valid_lens_tensor).to(self.device, torch.int64).contiguous()
+        dev = self._dev
+        logits = _on(int8_logits, dev, torch.int8)
+        valid = _on(valid_lens_tensor, dev, torch.int64)
         if valid.shape != (self.B,):
             raise ValueError("valid_lens must have shape (batch,)")
-        lut = _lut_on(exp_lut, self.device)
-        with torch.cuda.device(self.device):
-            _hip.check(_hip.lib().sc_decode_step(
-                _hip.ptr(logits), _hip.ptr(lut), _hip.ptr(valid), int(t), self.B, self._state,
-                _hip.ptr(self.comp_words), _hip.ptr(self.symbols_out), _hip.stream_ptr()))
+        lut = _lut_on(exp_lut, dev)
+        _launch(dev, _hip.lib().sc_decode_step, _hip.ptr(logits), _hip.ptr(lut), _hip.ptr(valid), int(t), self.B, self._state,
+                _hip.ptr(self.comp_words), _hip.ptr(self.symbols_out))
         return self.symbols_out
 
     def check(self):
