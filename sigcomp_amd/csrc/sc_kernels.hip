@@ -1207,6 +1207,7 @@ constexpr int64_t FED_SET_AIM = 6;   // tiles per feeder set while CUs are free
 // longer, bounds the step.
 static FedPlan fed_plan_of(int64_t n, int64_t cu, int64_t xch_cap, int rt_only) {
     FedPlan best{};
+    if (n < 1) return best;   // (no chunks left over: no sets to divide them by)
     for (int rt = 1; rt <= FED_RT_MAX; ++rt) {
         const int64_t heads = (n + 32 * rt - 1) / (32 * rt), tiles = heads * rt;
         if ((rt_only && rt != rt_only) || tiles > FED_MAX_TILES || fed_bytes(tiles) > xch_cap) continue;
