@@ -252,7 +252,8 @@ int64_t sc_decompress_workspace_bytes(int64_t n_chunks);
  * descending length (as QuantMLPCompression passes them) give the shortest
  * schedule: the shortest chunks are then left over after the full waves of
  * workgroups and follow the shortest chunks of the last full wave in the
- * same rows.  A launch of at most 256 tiles of 32 chunks (on 256 CUs) runs
+ * same rows, or, with lengths_host, groups of chunks take turns on the CUs, a
+ * launch of steps at a time, where the plan finds that cheaper.  A launch of at most 256 tiles of 32 chunks (on 256 CUs) runs
  * fed: one workgroup per tile or pair of tiles decodes it, sets of 16 more
  * compute layer 0 of the next step for up to 32 tiles each, and they wait for
  * each other every step

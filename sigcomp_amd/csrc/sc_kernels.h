@@ -62,10 +62,14 @@ void launch_ctx_two(const ModelDev &M, hipStream_t s, const int64_t *ctx, int64_
                     int32_t *status, uint8_t *feat);
 void launch_compress_mlp(const ModelDev &M, unsigned grid, hipStream_t s, const uint8_t *tokens, int64_t n_chunks,
                          const int32_t *tile_start, const int4 *desc, int64_t max_desc, uint2 *pairs);
+// The first n_first workgroups decode steps t_begin .. t_end of the groups of
+// 32 RT chunks from g_first on, the others the next t_end - t_begin steps of
+// the groups from 0 on.
 template <int RT>
 void launch_decompress(const ModelDev &M, unsigned grid, hipStream_t s, const uint32_t *words, const int64_t *woff,
                        const int32_t *wcnt, const int32_t *len, int64_t count, uint8_t *tokens, const int64_t *toff,
-                       int32_t *st, DecState *state, int32_t t_begin, int32_t t_end, int64_t n_second);
+                       int32_t *st, DecState *state, int32_t t_begin, int32_t t_end, int64_t n_second, int32_t g_first,
+                       int32_t n_first);
 // The split decode of `groups` 32-chunk groups with p = 4 or 8 workgroups
 // each (pipelined per-tensor core only): a cooperative launch of groups * p
 // workgroups, so that all are resident at once; returns the launch's error
@@ -785,9 +789,9 @@ __global__ __launch_bounds__(THREADS, 1) void k_decompress(ModelDev M, const uin
                                                            int64_t n_chunks, uint8_t *__restrict__ tokens,
                                                            const int64_t *__restrict__ tok_off,
                                                            int32_t *__restrict__ status,
-                                                           DecState *__restrict__ state, int32_t t_begin,
-                                                           int32_t t_end, int64_t n_second, uint8_t *xch,
-                                                           int32_t spin_max) {
+                                                           DecState *__restrict__ state, int32_t t_first,
+                                                           int32_t t_first_end, int64_t n_second, int32_t g_first,
+                                                           int32_t n_first, uint8_t *xch, int32_t spin_max) {
     // Rows n_chunks - n_second .. n_chunks - 1 each decode a second chunk
     // after their first one ends: row c continues with chunk
     // 2 * n_chunks - 1 - c (the n_second chunks after the launch's own, in
@@ -827,7 +831,11 @@ __global__ __launch_bounds__(THREADS, 1) void k_decompress(ModelDev M, const uin
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int q4 = lane >> 4, u = lane & 15;
     const int slice = P > 1 ? (int)(blockIdx.x % P) : 0;
-    const int64_t group = blockIdx.x / P, c0 = group * R;
+    // (launch_decompress: two runs of groups, the second one segment ahead)
+    const bool ahead = P == 1 && (int32_t)blockIdx.x >= n_first;
+    const int64_t group = P > 1 ? blockIdx.x / P : ahead ? blockIdx.x - n_first : blockIdx.x + g_first, c0 = group * R;
+    const int32_t t_begin = ahead ? t_first_end : t_first;
+    const int32_t t_end = ahead ? t_first_end + (t_first_end - t_first) : t_first_end;
     const bool writer = slice == 0;   // the workgroup that writes tokens, status and state
     if (threadIdx.x == 0) {
         s_maxlen = 0;

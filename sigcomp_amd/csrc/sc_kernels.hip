@@ -1262,6 +1262,74 @@ static void host_len_stats(const int32_t *len, int64_t n, int64_t g0, int64_t G,
     }
 }
 
+// Rotating decode launches.  A chunk's steps are serial, but its coder state
+// lies in memory between step segments, so the workgroups of a launch need
+// not be those of the last one: where the chunks are no whole number of full
+// waves, the groups of 32 rt chunks take turns on the CUs, a segment at a
+// time (640 tiles of 2,048 steps on 256 CUs: ten full launches of 64-chunk
+// workgroups, where a wave of 64-chunk workgroups for all 2,048 steps left
+// 128 tiles to a second one).  A launch takes the next cu items of the order
+// (segment, group): groups g_first .. of segment k and, when those run out,
+// the first groups of segment k + 1, none of which runs twice in a launch.
+// Measured: 20,480 chunks of 2,048 tokens, 216.3 ms as full waves and a fed
+// tail, 200.5 ms rotating.
+struct RotLaunch {
+    int32_t k, g_first, n_first, n_ahead;
+};
+struct RotPlan {
+    int rt = 0;
+    int64_t seg = 0, cost = INT64_MAX;   // DEC_STEP_COST's unit
+    std::vector<RotLaunch> launches;
+};
+// A launch's time beyond its steps (tables staged, the first layer 0 and the
+// last epilogue alone, the workgroups' drift), in DEC_STEP_COST's unit.
+constexpr int64_t DEC_LAUNCH_COST = 400;
+
+static RotPlan rot_plan(const int32_t *len, int64_t n, int64_t cu) {
+    RotPlan best;
+    for (int rt = 1; rt <= RT_TILE; ++rt) {
+        const int64_t R = 32 * rt, G = (n + R - 1) / R;
+        if (G <= cu / 2) continue;
+        std::vector<int32_t> longest((size_t)G, 0);   // of the group and all after it
+        for (int64_t i = n - 1, m = 0; i >= 0; --i) {
+            m = std::max<int64_t>(m, len[i]);
+            longest[(size_t)(i / R)] = (int32_t)m;
+        }
+        for (int64_t seg = DEC_SEG_STEPS; seg >= WIN; seg /= 2) {
+            const int64_t K = std::max<int64_t>(1, (longest[0] + seg - 1) / seg);
+            // groups with steps in segment k (k does not fall from call to call)
+            int64_t act = G;
+            auto active = [&](int64_t k) {
+                int64_t a = act;
+                while (k > 0 && a > 0 && longest[(size_t)a - 1] <= k * seg) --a;
+                return a;
+            };
+            RotPlan p;
+            p.rt = rt;
+            p.seg = seg;
+            p.cost = 0;
+            for (int64_t k = 0, g = 0; k < K;) {
+                act = active(k);
+                const int64_t n_first = std::min(cu, act - g);
+                const bool ends = g + n_first == act;
+                const int64_t n_ahead = ends && k + 1 < K ? std::min({cu - n_first, active(k + 1), g}) : 0;
+                int64_t steps = std::min<int64_t>(seg, longest[(size_t)g] - k * seg);
+                if (n_ahead) steps = std::max(steps, std::min<int64_t>(seg, longest[0] - (k + 1) * seg));
+                p.cost += steps * DEC_STEP_COST[rt] + DEC_LAUNCH_COST;
+                p.launches.push_back({(int32_t)k, (int32_t)g, (int32_t)n_first, (int32_t)n_ahead});
+                g = ends ? n_ahead : g + n_first;
+                k += ends;
+                if (k < K && g == active(k)) {   // the segment's groups all ran ahead
+                    ++k;
+                    g = 0;
+                }
+            }
+            if (p.cost < best.cost) best = std::move(p);
+        }
+    }
+    return best;
+}
+
 // The decode of sc_decompress_chunks with its buffers given: `state` holds
 // DecState for n_chunks rows, `stat_dev` 4 int32 (used only when
 // lengths_host is NULL), `xch` xch_cap bytes of exchange buffers for a fed
@@ -1382,6 +1450,25 @@ static int decompress_run(const sc_model *m, const uint32_t *words, const int64_
     const bool pair = can_pair && (int64_t)std::max(0, pair_max - group_max) * DEC_STEP_COST[rt_last] <
                                       (int64_t)left_max * left_cost;
     const int64_t maxlen = std::max(len_max, pair ? pair_max : 0);
+    // The plan's cost against rotating launches': its launches' longest
+    // chunks' steps, the pairs' or the leftover launch's.  Rotating launches
+    // have to be 2% cheaper, which is what the step costs are good to.  (They
+    // need the lengths here, so a call without lengths_host keeps the plan.)
+    RotPlan rot;
+    // (Chunks beyond 2**20 tokens keep the plan too: the host lists every launch.)
+    if (m->dev.pipe == CORE_PIPE_UNI && units >= 1 && lengths_host && len_max <= (1 << 20) && !rt_cap && !plan_env &&
+        !seg_env && !pair_env && !split_env) {
+        int64_t cost = pair ? (int64_t)std::max(0, pair_max - group_max) * DEC_STEP_COST[rt_last]
+                            : left ? (int64_t)left_max * left_cost : 0;
+        const int32_t *at = lengths_host;
+        for (int rt : plan) {
+            const int32_t *end = at + rt * 32 * cu;
+            cost += (int64_t)std::max(0, *std::max_element(at, end)) * DEC_STEP_COST[rt];
+            at = end;
+        }
+        rot = rot_plan(lengths_host, n_chunks, cu);
+        if (rot.cost > cost / 50 * 49) rot.rt = 0;
+    }
     if (const char *log = getenv("SC_HIP_DEC_LOG"); log && std::strcmp(log, "1") == 0) {
         std::string rts;
         for (int rt : plan) rts += (rts.empty() ? "" : ",") + std::to_string(rt);
@@ -1392,6 +1479,21 @@ static int decompress_run(const sc_model *m, const uint32_t *words, const int64_
                      (long long)n_chunks, (long long)cu, rts.c_str(), (long long)left,
                      left == 0 ? "none" : pair ? "paired" : pl == 8 ? "split launch p8" : pl == 4 ? "split launch p4" : "launch",
                      (long long)maxlen, (long long)seg, fl.heads, fl.sets, FED_SLICES, fl.rt);
+        if (rot.rt)
+            std::fprintf(stderr, "sc_decompress_chunks: in its place rotating launches: rt %d seg %lld launches %zu\n", rot.rt,
+                         (long long)rot.seg, rot.launches.size());
+    }
+    if (rot.rt) {
+        auto *launch = rot.rt == 1 ? launch_decompress<1> : rot.rt == 2 ? launch_decompress<2>
+                     : rot.rt == 3 ? launch_decompress<3> : launch_decompress<4>;
+        for (const RotLaunch &l : rot.launches) {
+            const int64_t t0 = l.k * rot.seg, t1 = t0 + rot.seg;
+            launch(m->dev, (unsigned)(l.n_first + l.n_ahead), s, words, word_off, word_cnt, lengths, n_chunks, tokens,
+                   tok_off, status, state, (int32_t)t0, (int32_t)t1, 0, l.g_first, l.n_first);
+            const int rc = check_launch("k_decompress (rotating)");
+            if (rc) return rc;
+        }
+        return SC_OK;
     }
     int64_t start = 0;
     size_t step = 0;
@@ -1464,7 +1566,8 @@ static int decompress_run(const sc_model *m, const uint32_t *words, const int64_
             switch (rt) {
 #define SC_DEC_CASE(N)                                                                                        \
     case N:                                                                                                   \
-        launch_decompress<N>(m->dev, grid, s, wds, woff, wcnt, len, count, tokens, toff, st, ds, t0, t1, n_second);       \
+        launch_decompress<N>(m->dev, grid, s, wds, woff, wcnt, len, count, tokens, toff, st, ds, t0, t1, n_second, 0,     \
+                             (int32_t)grid);                                                                              \
         break;
                 SC_DEC_CASE(1)
                 SC_DEC_CASE(2)
