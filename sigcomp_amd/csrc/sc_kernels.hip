@@ -83,7 +83,9 @@ __global__ __launch_bounds__(256) void k_tile_table(const int64_t *__restrict__ 
 // words that will be all ones or, after a carry, zeros); here every word goes
 // out at once and a carry out of `lower` is added to the words already
 // written, which gives the same words: a held-back word is 0xFFFFFFFF until
-// the carry turns it into 0.
+// the carry turns it into 0.  (A chunk whose words do not fit its capacity
+// is coded again with the words held back, which leaves the words committed
+// before the step that does not fit and their count.)
 //
 // A step depends on the last one, so the kernel is one latency chain per
 // chunk: about twenty instructions per step, with the pairs loaded
@@ -124,8 +126,11 @@ __global__ __launch_bounds__(64) void k_encode_pairs(const uint2 *__restrict__ p
         ++pos;
     };
     auto carry = [&] {
-        for (int32_t i = pos - 1; i >= 0; --i)
-            if (i < cap && ++out[i] != 0) break;
+        // (past the capacity nothing is carried: the chunk is coded again,
+        // and each walk back over words that are not there would be as long
+        // as all of them)
+        for (int32_t i = pos <= cap ? pos - 1 : -1; i >= 0; --i)
+            if (++out[i] != 0) break;
     };
     auto step = [&](const uint2 &x) __attribute__((always_inline)) {
         const uint64_t scale = range >> 24;
@@ -161,8 +166,16 @@ __global__ __launch_bounds__(64) void k_encode_pairs(const uint2 *__restrict__ p
         put((uint32_t)(point >> 32));
         if ((uint32_t)((lower + range) >> 32) == (uint32_t)(point >> 32)) put(0u);
     }
-    word_cnt[c] = min(pos, cap);
-    status[c] = pos > cap ? SC_STATUS_CAPACITY : SC_STATUS_OK;
+    int st = SC_STATUS_OK;
+    if (__builtin_expect(pos > cap, 0)) {
+        EncState s{0ull, ~0ull, 0, 0u, 0};
+        for (int32_t t = 0; t < L && !st; ++t)
+            if (enc_step(s, p[t].x, p[t].y, out, cap)) st = SC_STATUS_CAPACITY;
+        if (!st && L > 0 && enc_seal(s, out, cap)) st = SC_STATUS_CAPACITY;
+        pos = s.pos;
+    }
+    word_cnt[c] = pos;
+    status[c] = st;
 }
 
 // Length statistics for the decode plan, each max(0, ...), one workgroup of
