@@ -913,14 +913,15 @@ __global__ __launch_bounds__(THREADS, 1) void k_decompress(ModelDev M, const uin
     load_lut_lds(M.lut, s_lut);
     if constexpr (P > 1) split_params_init(M, s_par, split_ntile<P>(slice, wave), wave, lane);
     else mlp_tile_init<CORE>(M, s_par, wave, lane);
-    // Rows past the last chunk never write their ring: without this fill
-    // their layer-0 reads gather from whatever addresses the LDS held
-    // (unaligned ones among them, which take several LDS passes each).  A
-    // group of 10 chunks decoded at 34.7 us per split step, a full group
-    // (no such rows) at 25.0.
+    // Every slot of the ring starts as a table address: rows past the last
+    // chunk and rows whose chunk has ended (here, or in an earlier segment)
+    // write no further ones, and their layer-0 reads would gather from
+    // whatever the LDS held (unaligned addresses among them, which take
+    // several LDS passes each).
     if constexpr (PIPE) {
-        for (int i = threadIdx.x; i < R * WIN; i += THREADS)
-            if (c0 + i % R >= n_chunks) s_apos[i] = (uint16_t)emb_off(SOS, 0);
+        static_assert(R * WIN % 8 == 0, "whole 16-byte pieces");
+        const int sos = emb_off(SOS, 0) * 0x10001;
+        for (int i = threadIdx.x; i < R * WIN / 8; i += THREADS) ((v4i *)s_apos)[i] = v4i{sos, sos, sos, sos};
     }
     __syncthreads();
     if (t_begin > 0) {
