@@ -21,6 +21,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cstdlib>
 #include <string>
 
 #include "sc_fed.h"
@@ -233,7 +234,7 @@ __global__ __launch_bounds__(256) void k_gen_dec_status(const DecState *__restri
 //
 // Models whose activations fit the LDS (gen_fused_lds below: every width of
 // a layer up to about 1,500, an embedding width that is a multiple of 16)
-// run fused: a workgroup keeps 32 rows on chip from the token windows to the
+// run fused, but for few rows of wide ones (runs_fused below): a workgroup keeps 32 rows on chip from the token windows to the
 // logits, streams each layer's weights once per 32 rows, and ends with what
 // the call wants of the logits.  The decoder loops over its steps inside
 // one launch.  One launch per stage cost seven launches a step (57 us for 64
@@ -246,6 +247,9 @@ enum GenOut { GEN_LOGITS = 0, GEN_CDF = 1, GEN_PAIRS = 2, GEN_DECODE = 3 };
 constexpr int GEN_LDS = 156 * 1024;
 constexpr int GEN_BLK = 8;          // k-tiles per block of a layer's loop
 constexpr int GEN_MAX_WINDOW = 256;
+// A compress call in separate launches against the fused one, beyond what
+// their MLPs take (measured on seven models, 20 to 70 us)
+constexpr int GEN_COMPRESS_US = 50;
 
 // LDS of a fused workgroup, byte offsets (all multiples of 16)
 struct GenLds {
@@ -625,12 +629,46 @@ GenLds gen_fused_lds(const ModelDev &M) {
     return P;
 }
 
-// Workgroups of a fused launch over `tiles` 32-row tiles: one per CU.
-unsigned fused_grid(int64_t tiles) {
+int n_cu() {
     int dev = 0, cu = 0;
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
         cu = 256;
-    return (unsigned)std::max<int64_t>(1, std::min<int64_t>(tiles, cu));
+    return std::max(cu, 1);
+}
+
+// Workgroups of a fused launch over `tiles` 32-row tiles: one per CU.
+unsigned fused_grid(int64_t tiles) { return (unsigned)std::max<int64_t>(1, std::min<int64_t>(tiles, n_cu())); }
+
+// Whether a call whose MLP takes `rows` rows at a time runs fused.  A fused
+// workgroup streams all weights through its CU (88 GB/s) for its 32 rows; the
+// separate launches spread a layer's n-tiles over the device, but each waits
+// for its k-tiles one after the other and their rows go through memory.  So
+// few rows of a model with wide layers are cheaper in separate launches:
+// 16 chunks of a 64 x 128 -> 1024 x 6 -> 256 model take 138 us a step so and
+// 188 fused, of a 64 x 16 -> 1400 x 4 -> 256 model 61 and 132; 4,096 chunks
+// 797 and 183, 198 and 126.  The costs in us are least-squares fits to the
+// decode steps of eighteen models (82 thousand to 14 million weights) at 1
+// to 4,096 chunks, of which they choose the faster form every time.
+// `once_us` is what the call's first separate launches cost beyond a step.
+// SC_HIP_GEN_FUSED = 0 or 1 forces one form (comparisons and tests of both).
+bool runs_fused(const ModelDev &M, const GenLds &P, int64_t rows, int once_us) {
+    if (!P.bytes) return false;
+    const char *env = getenv("SC_HIP_GEN_FUSED");
+    if (env && (env[0] == '0' || env[0] == '1') && env[1] == 0) return env[0] == '1';
+    double kts = 0, weights = 0, passes = 0, streamed = 0;
+    for (int i = 0; i < M.n_layers; ++i) {
+        // (a wave streams two n-tiles per pass, whether or not it has two)
+        const int nt = (M.layer[i].n + 31) / 32, ps = (nt + 2 * WAVES - 1) / (2 * WAVES);
+        kts += M.layer[i].kt;
+        weights += (double)nt * M.layer[i].kt * 1024;
+        passes += ps;
+        streamed += (double)ps * 2 * WAVES * M.layer[i].kt * 1024;
+    }
+    const int64_t tiles = (rows + 31) / 32, cu = n_cu();
+    const double fused = (double)((tiles + cu - 1) / cu) * (1.7 + 0.35 * M.n_layers + 1.32 * passes + streamed / 88.2e3);
+    const double separate = once_us + 2.51 * (M.n_layers + 2) + 0.206 * kts + 0.192 * M.emb_dim +
+                            (double)rows * ((double)M.window * M.emb_dim / 195e3 + weights / 379e6);
+    return fused <= separate;
 }
 
 // Widest padded layer input / output of the model (bytes per row).
@@ -704,7 +742,7 @@ hipError_t gen_mlp(const ModelDev &M, const GenRows &g, int64_t rows, int8_t *X0
 
 int gen_mlp_forward(const ModelDev &M, const int64_t *ctx, int64_t rows, int8_t *logits, int32_t *cdf,
                     int32_t *status, hipStream_t s, std::string &err) {
-    if (const GenLds P = gen_fused_lds(M); P.bytes) {
+    if (const GenLds P = gen_fused_lds(M); runs_fused(M, P, rows, 0)) {
         GenArgs A{};
         A.ctx = ctx;
         A.logits = logits;
@@ -744,7 +782,7 @@ int gen_mlp_forward(const ModelDev &M, const int64_t *ctx, int64_t rows, int8_t 
 
 int gen_compress(const ModelDev &M, const uint8_t *tokens, const int32_t *tile_start, int64_t n_chunks,
                  const int4 *desc, int64_t max_tiles, uint2 *pairs, hipStream_t s, std::string &err) {
-    if (const GenLds P = gen_fused_lds(M); P.bytes) {
+    if (const GenLds P = gen_fused_lds(M); runs_fused(M, P, max_tiles * R_GEN_TILE, GEN_COMPRESS_US)) {
         GenArgs A{};
         A.tokens_in = tokens;
         A.desc = desc;
@@ -783,7 +821,7 @@ int gen_compress(const ModelDev &M, const uint8_t *tokens, const int32_t *tile_s
 int gen_decompress(const ModelDev &M, const uint32_t *words, const int64_t *word_off, const int32_t *word_cnt,
                    const int32_t *lengths, int64_t n_chunks, uint8_t *tokens, const int64_t *tok_off,
                    int32_t *status, DecState *state, int32_t max_len, hipStream_t s, std::string &err) {
-    if (const GenLds P = gen_fused_lds(M); P.bytes) {
+    if (const GenLds P = gen_fused_lds(M); runs_fused(M, P, n_chunks, 0)) {
         GenArgs A{};
         A.status = status;
         A.words = words;

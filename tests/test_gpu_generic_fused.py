@@ -1,7 +1,10 @@
 """GPU tests of the fused generic kernel: architectures at the edges of what
 it takes (embedding widths that are multiples of 16, windows that are no
 power of two, widths that are no multiple of 32, one and many layers) and
-just beyond it, against the oracle."""
+just beyond it, against the oracle; and which calls run in it instead of in
+separate launches."""
+
+import time
 
 import numpy as np
 import pytest
@@ -50,3 +53,49 @@ def test_round_trip_and_corrupt_chunk(arch, oracle_mod):
     enc[4] = b"\xff" * 8
     with pytest.raises(ValueError, match="chunk 4"):
         codec.decompress_chunks(enc, lengths)
+
+
+def _wide():
+    from sigcomp_amd.model_io import random_int_model
+    from sigcomp_amd.quant_mlp_export import QuantMLPCompression
+    m = random_int_model(seed=5, window=64, emb_dim=16, hidden=1400, n_hidden=4, per_channel=False)
+    return m, QuantMLPCompression(chunk_len=300, gpu=0, model=m)
+
+
+@pytest.mark.parametrize("fused", ["0", "1", None])
+def test_wide_model_in_both_forms(oracle_mod, monkeypatch, fused):
+    """A model with wide layers, whose small calls run in separate launches
+    and whose large ones run fused."""
+    if fused is not None:
+        monkeypatch.setenv("SC_HIP_GEN_FUSED", fused)
+    m, codec = _wide()
+    rng = np.random.default_rng(2)
+    om = oracle_mod.OracleModel(m)
+    ctx = rng.integers(0, 257, (2100, m.window)).astype(np.int64)
+    ref = oracle_mod.mlp_forward(om, ctx)
+    for rows in (1, 40, 2100):
+        got = codec.hip.forward_windows(torch.from_numpy(ctx[:rows]).cuda(), "logits").cpu().numpy()
+        assert np.array_equal(got, ref[:rows]), rows
+    lengths = [1, 31, 63, 64, 65, 100]
+    chunks = [rng.integers(0, 60, n).astype(np.uint8) for n in lengths]
+    enc = codec.compress_chunks(chunks)
+    assert enc == oracle_mod.compress_chunks(om, chunks)
+    assert all(np.array_equal(a, b) for a, b in zip(chunks, codec.decompress_chunks(enc, lengths)))
+
+
+def test_few_rows_of_a_wide_model_take_the_faster_form(monkeypatch):
+    """Sixteen chunks: 61 us a step in separate launches, 132 fused."""
+    _, codec = _wide()
+    tokens, lengths = np.random.default_rng(1).integers(0, 60, 16 * 96).astype(np.uint8), np.full(16, 96, np.int32)
+    words, off, cnt = (np.array(a) for a in codec.compress_flat(tokens, lengths))
+    best = {}
+    for form in ("0", "1", None):
+        monkeypatch.delenv("SC_HIP_GEN_FUSED", raising=False)
+        if form is not None:
+            monkeypatch.setenv("SC_HIP_GEN_FUSED", form)
+        for _ in range(4):
+            torch.cuda.synchronize()
+            start = time.perf_counter()
+            assert np.array_equal(codec.decompress_flat(words, off, cnt, lengths)[0], tokens)
+            best[form] = min(best.get(form, 1e9), time.perf_counter() - start)
+    assert best["1"] > 1.4 * best["0"] and best[None] < 1.2 * best["0"], best
