@@ -128,7 +128,8 @@ class HipModel:
                 res = torch.empty((rows, VOCAB_SIZE), dtype=torch.int8, device=self.device)
             else:
                 res = torch.empty((rows, VOCAB_SIZE + 1), dtype=torch.int32, device=self.device)
-            nbytes = int(_hip.lib().sc_mlp_forward_workspace_bytes(rows))
+            # (the other cores take no workspace)
+            nbytes = int(_hip.lib().sc_mlp_forward_workspace_bytes(rows)) if self.pipelined else 0
             ws = torch.empty(nbytes, dtype=torch.uint8, device=self.device) if nbytes else None
             to = (_hip.ptr(res), None) if out == "logits" else (None, _hip.ptr(res))
             _hip.check(_hip.lib().sc_mlp_forward_ws(self.handle, _hip.ptr(ctx), rows, *to, _hip.ptr(status),

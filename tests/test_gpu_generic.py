@@ -149,3 +149,15 @@ def test_generic_wide_model_batches_within_its_scratch_bound(oracle_mod):
     assert comp == oracle_mod.compress_chunks(om, chunks)
     back = codec.decompress_chunks(comp, [len(c) for c in chunks])
     assert all(np.array_equal(a, b) for a, b in zip(chunks, back))
+
+
+def test_forward_allocates_its_results_only(arch):
+    """The generic kernels take no workspace of the caller's: a call of few
+    rows allocates the status word and the result."""
+    _, m, codec = arch
+    ctx = torch.zeros((2, m.window), dtype=torch.int64, device="cuda")
+    codec.hip.forward_windows(ctx)
+    count = lambda: torch.cuda.memory_stats()["allocation.all.allocated"]
+    before = count()
+    codec.hip.forward_windows(ctx)
+    assert count() - before == 2
