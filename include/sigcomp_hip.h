@@ -55,9 +55,9 @@ extern "C" {
 #define SC_STATUS_CAPACITY 1        /* encoder output capacity exceeded (OverflowError) */
 #define SC_STATUS_INVALID_STREAM 2  /* decoder: scale == 0 or quantile >= 2**24 (ValueError) */
 #define SC_STATUS_BAD_TOKEN 3       /* context token outside [0, 256] (ValueError) */
-#define SC_STATUS_SYNC_TIMEOUT 4    /* decoder: the workgroups sharing a fed decode's layer 0
-                                       waited too long for each other (RuntimeError; tokens
-                                       unspecified) */
+#define SC_STATUS_SYNC_TIMEOUT 4    /* decoder: the workgroups sharing the layer 0 of a fed or split
+                                       decode of up to 64 tiles waited too long for each other
+                                       (RuntimeError; tokens unspecified) */
 
 #define SC_VOCAB 256
 #define SC_SOS 256
@@ -253,13 +253,15 @@ int64_t sc_decompress_workspace_bytes(int64_t n_chunks);
  * schedule: the shortest chunks are then left over after the full waves of
  * workgroups and follow the shortest chunks of the last full wave in the
  * same rows, or, with lengths_host, groups of chunks take turns on the CUs, a
- * launch of steps at a time, where the plan finds that cheaper.  A launch of at most 256 tiles of 32 chunks (on 256 CUs) runs
- * fed: one workgroup per tile or pair of tiles decodes it, sets of 16 more
- * compute layer 0 of the next step for up to 32 tiles each, and they wait for
- * each other every step
- * (a cooperative launch, so all are resident; a bounded wait,
- * SC_STATUS_SYNC_TIMEOUT when it expires), except
- * on a stream under graph capture.  Replaces
+ * launch of steps at a time, where the plan finds that cheaper.  A launch of
+ * at most 256 tiles of 32 chunks (on 256 CUs) runs fed: one workgroup per
+ * tile or pair of tiles decodes it, sets of 16 more compute layer 0 of the
+ * next step for up to 32 tiles each, and they wait for each other every step
+ * (a cooperative launch, so all are resident), except on a stream under graph
+ * capture.  The waits are bounded: when one expires, as other streams'
+ * kernels can cause by holding CUs for half a second, a launch of up to 64
+ * tiles reports SC_STATUS_SYNC_TIMEOUT for its chunks and a larger one
+ * decodes them again without waiting.  Replaces
  * QuantMLPCompression.decompress_chunks / _decompress_chunks_gpu
  * (quant_mlp_export.py:325-377); output equals
  * CPUQuantMLPCompression.decompress_chunks (cpu_compression.py:259-332). */

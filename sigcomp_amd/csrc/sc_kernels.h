@@ -64,12 +64,13 @@ void launch_compress_mlp(const ModelDev &M, unsigned grid, hipStream_t s, const 
                          const int32_t *tile_start, const int4 *desc, int64_t max_desc, uint2 *pairs);
 // The first n_first workgroups decode steps t_begin .. t_end of the groups of
 // 32 RT chunks from g_first on, the others the next t_end - t_begin steps of
-// the groups from 0 on.
+// the groups from 0 on.  late_only (RT = 1, pipelined per-tensor core): only
+// groups with a chunk whose status is SC_STATUS_SYNC_TIMEOUT.
 template <int RT>
 void launch_decompress(const ModelDev &M, unsigned grid, hipStream_t s, const uint32_t *words, const int64_t *woff,
                        const int32_t *wcnt, const int32_t *len, int64_t count, uint8_t *tokens, const int64_t *toff,
                        int32_t *st, DecState *state, int32_t t_begin, int32_t t_end, int64_t n_second, int32_t g_first,
-                       int32_t n_first);
+                       int32_t n_first, bool late_only);
 // The split decode of `groups` 32-chunk groups with p = 4 or 8 workgroups
 // each (pipelined per-tensor core only): a cooperative launch of groups * p
 // workgroups, so that all are resident at once; returns the launch's error
@@ -837,6 +838,13 @@ __global__ __launch_bounds__(THREADS, 1) void k_decompress(ModelDev M, const uin
     const int32_t t_begin = ahead ? t_first_end : t_first;
     const int32_t t_end = ahead ? t_first_end + (t_first_end - t_first) : t_first_end;
     const bool writer = slice == 0;   // the workgroup that writes tokens, status and state
+    if constexpr (P == 1 && RT == 1 && PIPE) {
+        // launch_decompress' late_only
+        if (spin_max < 0) {
+            const int64_t c = c0 + threadIdx.x;
+            if (!__syncthreads_or(threadIdx.x < R && c < n_chunks && status[c] == SC_STATUS_SYNC_TIMEOUT)) return;
+        }
+    }
     if (threadIdx.x == 0) {
         s_maxlen = 0;
         s_xerr = 0;

@@ -1502,7 +1502,7 @@ static int decompress_run(const sc_model *m, const uint32_t *words, const int64_
         for (const RotLaunch &l : rot.launches) {
             const int64_t t0 = l.k * rot.seg, t1 = t0 + rot.seg;
             launch(m->dev, (unsigned)(l.n_first + l.n_ahead), s, words, word_off, word_cnt, lengths, n_chunks, tokens,
-                   tok_off, status, state, (int32_t)t0, (int32_t)t1, 0, l.g_first, l.n_first);
+                   tok_off, status, state, (int32_t)t0, (int32_t)t1, 0, l.g_first, l.n_first, false);
             const int rc = check_launch("k_decompress (rotating)");
             if (rc) return rc;
         }
@@ -1544,6 +1544,19 @@ static int decompress_run(const sc_model *m, const uint32_t *words, const int64_
             if (e == hipSuccess) {
                 rc = check_launch("k_decompress_fed");
                 if (rc) return rc;
+                // Callers of up to XCH_MAX_GROUPS groups have always seen
+                // waits that time out (when other streams' kernels hold
+                // CUs) and decode again; larger batches never waited
+                // between workgroups before they ran fed.  Their groups that
+                // timed out are decoded again here: one launch whose
+                // workgroups look at their statuses and end (5 us beside
+                // at least 20 a step).
+                if (grid > XCH_MAX_GROUPS) {
+                    launch_decompress<1>(m->dev, grid, s, wds, woff, wcnt, len, count, tokens, toff, st, nullptr, 0,
+                                         INT32_MAX, 0, 0, (int32_t)grid, true);
+                    rc = check_launch("k_decompress (timed out groups)");
+                    if (rc) return rc;
+                }
                 start += count;
                 continue;
             }
@@ -1580,7 +1593,7 @@ static int decompress_run(const sc_model *m, const uint32_t *words, const int64_
 #define SC_DEC_CASE(N)                                                                                        \
     case N:                                                                                                   \
         launch_decompress<N>(m->dev, grid, s, wds, woff, wcnt, len, count, tokens, toff, st, ds, t0, t1, n_second, 0,     \
-                             (int32_t)grid);                                                                              \
+                             (int32_t)grid, false);                                                                       \
         break;
                 SC_DEC_CASE(1)
                 SC_DEC_CASE(2)

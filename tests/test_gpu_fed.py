@@ -119,3 +119,42 @@ def test_smaller_workspace_runs_split(codec, monkeypatch, capfd):
     log = capfd.readouterr().err
     assert "split launch p8" in log and "fed 0+0" in log
     assert not status.any().item() and np.array_equal(out.cpu().numpy(), tokens)
+
+
+@pytest.mark.parametrize("n,rt", [(2049, "1"), (4171, "2")])
+def test_large_fed_decode_never_reports_a_timeout(codec, monkeypatch, n, rt):
+    """Batches of more than 64 tiles never waited between workgroups before
+    they ran fed: where a wait expires (here each at once, SC_HIP_DEC_SPIN=0)
+    the call decodes the tiles again without waiting, so that its tokens are
+    right, every status is written and a corrupt chunk, and only it, is
+    reported as such."""
+    from sigcomp_amd import _hip
+    rng = np.random.default_rng(n)
+    tokens, lengths, words, off, cnt = _chunks(codec, rng.integers(0, 70, n), n)
+    bad = int(np.argmax(lengths))
+    words = np.concatenate([words, np.full(2, 0xFFFFFFFF, np.uint32)])
+    off[bad], cnt[bad] = len(words) - 2, 2
+    toff = np.concatenate([[0], np.cumsum(lengths[:-1], dtype=np.int64)]).astype(np.int64)
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    dev = [d(words.view(np.int32)), d(off), d(cnt), d(lengths), d(toff)]
+    out = torch.zeros(len(tokens), dtype=torch.uint8, device="cuda")
+    status = torch.full((n,), -1, dtype=torch.int32, device="cuda")
+    ws = codec._decompress_workspace(n)
+    monkeypatch.setenv("SC_HIP_DEC_FED", rt)
+    want = np.zeros(n, np.int32)
+    want[bad] = _hip.SC_STATUS_INVALID_STREAM
+    keep = np.ones(len(tokens), bool)
+    keep[toff[bad]:toff[bad] + lengths[bad]] = False
+    for spin in ("0", None):
+        if spin is None:
+            monkeypatch.delenv("SC_HIP_DEC_SPIN")
+        else:
+            monkeypatch.setenv("SC_HIP_DEC_SPIN", spin)
+        out.zero_()
+        status.fill_(-1)
+        _hip.check(_hip.lib().sc_decompress_chunks(
+            codec.hip.handle, *[x.data_ptr() for x in dev[:4]], n, out.data_ptr(), dev[4].data_ptr(), status.data_ptr(),
+            lengths.ctypes.data, ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream))
+        torch.cuda.synchronize()
+        assert np.array_equal(status.cpu().numpy(), want), spin
+        assert np.array_equal(out.cpu().numpy()[keep], tokens[keep]), spin
