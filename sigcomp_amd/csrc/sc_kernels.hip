@@ -1468,9 +1468,10 @@ static int decompress_run(const sc_model *m, const uint32_t *words, const int64_
     // have to be 2% cheaper, which is what the step costs are good to.  (They
     // need the lengths here, so a call without lengths_host keeps the plan.)
     RotPlan rot;
+    const char *rot_env = getenv("SC_HIP_DEC_ROT");   // "0": never rotate (comparisons)
     // (Chunks beyond 2**20 tokens keep the plan too: the host lists every launch.)
     if (m->dev.pipe == CORE_PIPE_UNI && units >= 1 && lengths_host && len_max <= (1 << 20) && !rt_cap && !plan_env &&
-        !seg_env && !pair_env && !split_env) {
+        !seg_env && !pair_env && !split_env && !(rot_env && std::strcmp(rot_env, "0") == 0)) {
         int64_t cost = pair ? (int64_t)std::max(0, pair_max - group_max) * DEC_STEP_COST[rt_last]
                             : left ? (int64_t)left_max * left_cost : 0;
         const int32_t *at = lengths_host;
@@ -1482,19 +1483,22 @@ static int decompress_run(const sc_model *m, const uint32_t *words, const int64_
         rot = rot_plan(lengths_host, n_chunks, cu);
         if (rot.cost > cost / 50 * 49) rot.rt = 0;
     }
-    if (const char *log = getenv("SC_HIP_DEC_LOG"); log && std::strcmp(log, "1") == 0) {
-        std::string rts;
-        for (int rt : plan) rts += (rts.empty() ? "" : ",") + std::to_string(rt);
-        const int64_t rest_last = units == 0 ? n_chunks : pair ? 0 : left;
-        const int pl = rest_last ? split_p(rest_last) : 0;
-        const FedPlan fl = rest_last ? fed_plan(rest_last) : FedPlan{};
-        std::fprintf(stderr, "sc_decompress_chunks: chunks %lld cu %lld plan [%s] leftover %lld %s steps %lld seg %lld fed %d+%dx%d rt %d\n",
-                     (long long)n_chunks, (long long)cu, rts.c_str(), (long long)left,
-                     left == 0 ? "none" : pair ? "paired" : pl == 8 ? "split launch p8" : pl == 4 ? "split launch p4" : "launch",
-                     (long long)maxlen, (long long)seg, fl.heads, fl.sets, FED_SLICES, fl.rt);
-        if (rot.rt)
-            std::fprintf(stderr, "sc_decompress_chunks: in its place rotating launches: rt %d seg %lld launches %zu\n", rot.rt,
-                         (long long)rot.seg, rot.launches.size());
+    if (const char *log = getenv("SC_HIP_DEC_LOG"); log && std::strcmp(log, "1") == 0) {   // what is launched
+        if (rot.rt) {
+            std::fprintf(stderr, "sc_decompress_chunks: chunks %lld cu %lld rotating launches: rt %d steps %lld seg %lld launches %zu\n",
+                         (long long)n_chunks, (long long)cu, rot.rt, (long long)len_max, (long long)rot.seg,
+                         rot.launches.size());
+        } else {
+            std::string rts;
+            for (int rt : plan) rts += (rts.empty() ? "" : ",") + std::to_string(rt);
+            const FedPlan fl = pair ? FedPlan{} : fed_plan(left);
+            const int pl = split_p(left);
+            std::fprintf(stderr, "sc_decompress_chunks: chunks %lld cu %lld plan [%s] leftover %lld %s steps %lld seg %lld fed %d+%dx%d rt %d\n",
+                         (long long)n_chunks, (long long)cu, rts.c_str(), (long long)left,
+                         left == 0 ? "none" : pair ? "paired" : fl.heads ? "fed launch" : pl == 8 ? "split launch p8"
+                         : pl == 4 ? "split launch p4" : "launch",
+                         (long long)maxlen, (long long)seg, fl.heads, fl.sets, FED_SLICES, fl.rt);
+        }
     }
     if (rot.rt) {
         auto *launch = rot.rt == 1 ? launch_decompress<1> : rot.rt == 2 ? launch_decompress<2>

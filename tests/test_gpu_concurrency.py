@@ -23,7 +23,8 @@ def _chunk_sets(rng):
     return big, small
 
 
-def test_two_streams_share_one_model(int_models, oracle_mod, oracle_models, monkeypatch, capfd):
+@pytest.mark.parametrize("split", ["8", None])
+def test_two_streams_share_one_model(int_models, oracle_mod, oracle_models, monkeypatch, capfd, split):
     if not torch.cuda.is_available():
         pytest.fail("GPU tests need a HIP device")
     from sigcomp_amd.quant_mlp_export import QuantMLPCompression
@@ -39,7 +40,10 @@ def test_two_streams_share_one_model(int_models, oracle_mod, oracle_models, monk
 
     capfd.readouterr()
     monkeypatch.setenv("SC_HIP_DEC_LOG", "1")
-    monkeypatch.delenv("SC_HIP_DEC_SPLIT", raising=False)
+    if split is None:
+        monkeypatch.delenv("SC_HIP_DEC_SPLIT", raising=False)
+    else:
+        monkeypatch.setenv("SC_HIP_DEC_SPLIT", split)
     results, errors = [None, None], []
     start = threading.Barrier(2, timeout=60)
 
@@ -64,7 +68,9 @@ def test_two_streams_share_one_model(int_models, oracle_mod, oracle_models, monk
         t.join(timeout=240)
     assert not any(t.is_alive() for t in threads), "a worker thread did not finish"
     assert not errors, errors
-    assert "split launch" in capfd.readouterr().err   # the small batch's decode ran split
+    log = capfd.readouterr().err   # split beside unsplit workgroups, or two fed decodes
+    small, big = ("split launch p8", "launch") if split else ("fed launch", "fed launch")
+    assert f"leftover 96 {small} steps" in log and f"leftover 2500 {big} steps" in log, log
     for k in range(2):
         for comp, back in results[k]:
             assert comp == want[k]

@@ -15,6 +15,8 @@
   archive bytes -> scan -> GPU decompress -> reassembly.
 """
 
+import re
+
 import numpy as np
 import pytest
 
@@ -100,9 +102,9 @@ def test_c2_full_launch_against_oracle(gpu, oracle_mod):
 
 
 def test_c1_full_config_split_decode_every_chunk_against_oracle(gpu, oracle_mod, capfd, monkeypatch):
-    """Config c1 (BASELINE.json's CPU case, 64 reads, 675 chunks) through the
-    HIP path: compress_flat, then decompress_flat, whose single launch of
-    22 groups of 32 chunks runs split (8 workgroups per group sharing layer
+    """The 64-read case (675 chunks) through the HIP path: compress_flat, then
+    decompress_flat, whose single launch of 22 groups of 32 chunks runs fed
+    and, with SC_HIP_DEC_SPLIT=8, split (8 workgroups per group sharing layer
     0, one exchange per step) over eight 256-step segments.  Every chunk's
     bytes equal the oracle's and every decoded chunk equals its input."""
     from sigcomp_amd import model_io, signal, synth
@@ -119,12 +121,16 @@ def test_c1_full_config_split_decode_every_chunk_against_oracle(gpu, oracle_mod,
     capfd.readouterr()
     monkeypatch.setenv("SC_HIP_DEC_LOG", "1")
     monkeypatch.delenv("SC_HIP_DEC_SEG", raising=False)
-    monkeypatch.delenv("SC_HIP_DEC_SPLIT", raising=False)
-    back, tok_off = codec.decompress_flat(words, woff, wcnt, lengths)
-    log = capfd.readouterr().err
-    assert "split launch p8" in log and "seg 256" in log, log
     assert int(lengths.max()) == 2048
-    assert np.array_equal(back, tokens)
+    for split in ("8", None):
+        if split is None:
+            monkeypatch.delenv("SC_HIP_DEC_SPLIT")
+        else:
+            monkeypatch.setenv("SC_HIP_DEC_SPLIT", split)
+        back, tok_off = codec.decompress_flat(words, woff, wcnt, lengths)
+        log = capfd.readouterr().err
+        assert ("split launch p8 steps 2048 seg 256" if split else "fed launch steps 2048") in log, log
+        assert np.array_equal(back, tokens), split
     ref = oracle_mod.compress_chunks(oracle_mod.OracleModel(codec.model), chunks)
     for i in range(len(chunks)):
         assert words[woff[i]:woff[i] + wcnt[i]].tobytes() == ref[i], i
@@ -164,12 +170,17 @@ def test_full_config_round_trip_and_oracle_bytes(gpu, oracle_mod, capfd, monkeyp
     capfd.readouterr()
     monkeypatch.setenv("SC_HIP_DEC_LOG", "1")
     monkeypatch.delenv("SC_HIP_DEC_SEG", raising=False)
-    back, tok_off = codec.decompress_flat(words, woff, wcnt, lengths)
-    log = capfd.readouterr().err
-    import re
-    m = re.search(r"steps (\d+) seg 256", log)        # at least eight 256-step launches
-    assert m and int(m.group(1)) >= 2048, log
-    assert np.array_equal(back, tokens)
+    for rot in ("0", None):                               # the plan of full waves, the default one
+        if rot is None:
+            monkeypatch.delenv("SC_HIP_DEC_ROT")
+        else:
+            monkeypatch.setenv("SC_HIP_DEC_ROT", rot)
+        back, tok_off = codec.decompress_flat(words, woff, wcnt, lengths)
+        log = capfd.readouterr().err
+        m = re.search(r"steps (\d+) seg (\d+)", log)      # at least eight launches of 256 steps
+        assert m and int(m.group(1)) >= 2048 and int(m.group(2)) <= 256, log
+        assert rot is None or ("plan [" in log and m.group(2) == "256"), log
+        assert np.array_equal(back, tokens), rot
     pick = _oracle_pick(lengths, _n_cu(), np.random.default_rng(11))
     assert len(pick) >= 64 and int(lengths[pick].max()) == 2048
     ref = oracle_mod.compress_chunks(oracle_mod.OracleModel(codec.model), [chunks[i] for i in pick])

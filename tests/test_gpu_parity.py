@@ -1,6 +1,8 @@
 """GPU parity: the gfx950 kernels against the reference golden vectors and the
 CPU oracle, bit-exact (integer / byte work has no tolerance)."""
 
+import re
+
 import numpy as np
 import pytest
 
@@ -507,7 +509,7 @@ def test_full_symbol_range_against_oracle(codecs, oracle_mod, oracle_models, mon
     """Tokens uniform over all 256 symbols (most of them rare under the
     model: frequencies at the floor of 1, ~3 bytes of stream per token), and
     chunks of only 255 or only 0: every chunk's bytes equal the oracle's and
-    both the persistent and the split decode return the tokens."""
+    the persistent, the split and the fed decode return the tokens."""
     codec = codecs[name]
     rng = np.random.default_rng(256 + (name == "lossy"))
     lengths = rng.integers(1, 301, 200).astype(np.int32)
@@ -518,11 +520,8 @@ def test_full_symbol_range_against_oracle(codecs, oracle_mod, oracle_models, mon
     chunks[2][:] = 0
     comp = codec.compress_chunks(chunks)
     assert comp == oracle_mod.compress_chunks(oracle_models[name], chunks)
-    for split in ("0", None):
-        if split is None:
-            monkeypatch.delenv("SC_HIP_DEC_SPLIT", raising=False)
-        else:
-            monkeypatch.setenv("SC_HIP_DEC_SPLIT", split)
+    for split in ("0", "8", None):
+        _set_split(monkeypatch, split)
         back = codec.decompress_chunks(comp, list(lengths))
         assert all(np.array_equal(a, b) for a, b in zip(chunks, back)), split
 
@@ -681,15 +680,20 @@ def test_pipelined_core_selected_for_bundled_models(codecs):
     assert codecs["lossless"].hip.core == 2 and codecs["lossy"].hip.core == 2
 
 
-@pytest.mark.parametrize("pair", ["auto", "0"])
+@pytest.mark.parametrize("pair", ["auto", "0", "rotate"])
 @pytest.mark.parametrize("units,extra", [(2, 7), (3, 0), (4, 31), (5, 1), (6, 500)])
-def test_decompress_launch_plans(codecs, oracle_mod, oracle_models, monkeypatch, units, extra, pair):
+def test_decompress_launch_plans(codecs, oracle_mod, oracle_models, monkeypatch, capfd, units, extra, pair):
     """Chunk counts that fill `units` full waves of 32-chunk row tiles per CU
     (split by the launch planner into 64/96/128-chunk workgroup launches)
     plus leftover chunks, paired with the last launch's rows (auto) or in a
-    launch of their own (SC_HIP_DEC_PAIR=0); short random chunk lengths."""
+    launch of their own (SC_HIP_DEC_PAIR=0), without rotating launches
+    (SC_HIP_DEC_ROT=0); and whatever the plan is with them; short random
+    chunk lengths."""
+    if pair != "rotate":
+        monkeypatch.setenv("SC_HIP_DEC_ROT", "0")
     if pair == "0":
         monkeypatch.setenv("SC_HIP_DEC_PAIR", "0")
+    monkeypatch.setenv("SC_HIP_DEC_LOG", "1")
     n_cu = torch.cuda.get_device_properties(0).multi_processor_count
     n = units * 32 * n_cu + extra
     rng = np.random.default_rng(units * 1000 + extra)
@@ -697,7 +701,16 @@ def test_decompress_launch_plans(codecs, oracle_mod, oracle_models, monkeypatch,
     tokens = rng.integers(0, 50, int(lengths.sum())).astype(np.uint8)
     codec = codecs["lossless"]
     words, woff, wcnt = codec.compress_flat(tokens, lengths)
+    capfd.readouterr()
     back, tok_off = codec.decompress_flat(words, woff, wcnt, lengths)
+    log = capfd.readouterr().err
+    plan = re.search(r"plan \[([\d,]+)\] leftover (\d+) (\S+)", log)
+    if pair == "rotate":
+        assert plan or "rotating launches" in log, log
+    else:
+        assert sum(map(int, plan.group(1).split(","))) == units and int(plan.group(2)) == extra, log
+        if pair == "0" and extra:
+            assert plan.group(3) == "fed", log
     assert np.array_equal(back, tokens)
     sample = rng.choice(n, 16, replace=False)
     off = np.concatenate([[0], np.cumsum(lengths)[:-1]])
@@ -729,7 +742,7 @@ def test_decompress_greedy_plan_uses_160_chunk_workgroups(codecs, capfd, monkeyp
 def test_decompress_one_million_chunks(codecs, capfd, monkeypatch):
     """1,000,003 chunks of 1..6 tokens: a plan of many full-wave launches,
     the decode state buffer grown to a million rows, and the length
-    statistics over all of them."""
+    statistics over all of them; then whatever the default plan is."""
     rng = np.random.default_rng(7)
     n = 1_000_003
     lengths = rng.integers(1, 7, n).astype(np.int32)
@@ -738,9 +751,15 @@ def test_decompress_one_million_chunks(codecs, capfd, monkeypatch):
     words, woff, wcnt = codec.compress_flat(tokens, lengths)
     capfd.readouterr()
     monkeypatch.setenv("SC_HIP_DEC_LOG", "1")
-    back, _ = codec.decompress_flat(words, woff, wcnt, lengths)
-    assert "chunks 1000003" in capfd.readouterr().err
-    assert np.array_equal(back, tokens)
+    for rot in ("0", None):
+        if rot is None:
+            monkeypatch.delenv("SC_HIP_DEC_ROT")
+        else:
+            monkeypatch.setenv("SC_HIP_DEC_ROT", rot)
+        back, _ = codec.decompress_flat(words, woff, wcnt, lengths)
+        log = capfd.readouterr().err
+        assert "chunks 1000003" in log and (rot is None or "plan [" in log), log
+        assert np.array_equal(back, tokens), rot
 
 
 def _decode_direct(codec, words, woff, wcnt, lengths, host_lengths=True, ws_fill=None):
@@ -773,7 +792,10 @@ def _decode_direct(codec, words, woff, wcnt, lengths, host_lengths=True, ws_fill
 
 
 def _set_dec_env(monkeypatch, seg):
+    """The plan of full waves (no rotating launches), its log, and the steps
+    per launch."""
     monkeypatch.setenv("SC_HIP_DEC_LOG", "1")
+    monkeypatch.setenv("SC_HIP_DEC_ROT", "0")
     if seg is None:
         monkeypatch.delenv("SC_HIP_DEC_SEG", raising=False)
     else:
@@ -816,7 +838,7 @@ def test_decompress_rejects_pairing_of_long_leftovers(codecs, capfd, monkeypatch
     _set_dec_env(monkeypatch, None)
     back, _ = codec.decompress_flat(words, woff, wcnt, lengths)
     log = capfd.readouterr().err
-    assert "leftover 40 split launch" in log, log
+    assert "leftover 40 fed launch" in log, log
     assert np.array_equal(back, tokens)
 
 
@@ -886,10 +908,12 @@ def test_decompress_longest_row_is_a_pair_ending_on_a_segment_edge(codecs, capfd
         assert np.array_equal(back[s], tokens[s]), i
 
 
-def test_decompress_status_survives_later_segments(codecs, monkeypatch):
+@pytest.mark.parametrize("split,what", [("0", "launch"), ("8", "split launch p8"), ("4", "split launch p4")])
+def test_decompress_status_survives_later_segments(codecs, monkeypatch, capfd, split, what):
     """A corrupt chunk in a workgroup whose rows all end in the first 64-step
     launch keeps its status through the later launches another workgroup's
-    long chunk needs (those launches find nothing left to do there)."""
+    long chunk needs (those launches find nothing left to do there); unsplit
+    and split launches (a fed launch runs all steps)."""
     rng = np.random.default_rng(4)
     lengths = np.full(64, 10, np.int32)
     lengths[0] = 300
@@ -899,17 +923,28 @@ def test_decompress_status_survives_later_segments(codecs, monkeypatch):
     words = np.concatenate([words, np.full(2, 0xFFFFFFFF, np.uint32)])
     woff, wcnt = woff.copy(), wcnt.copy()
     woff[40], wcnt[40] = len(words) - 2, 2
-    monkeypatch.setenv("SC_HIP_DEC_SEG", "64")
+    _set_dec_env(monkeypatch, 64)
+    monkeypatch.setenv("SC_HIP_DEC_SPLIT", split)
     # a workspace holding another call's state (every row's "current chunk"
     # field nonzero): launches past a workgroup's rows must not read it
     for host_lengths, fill in ((True, None), (False, 1), (True, 255)):
+        capfd.readouterr()
         back, status, tok_off = _decode_direct(codec, words, woff, wcnt, lengths, host_lengths, fill)
+        assert f"leftover 64 {what} steps 300 seg 64" in capfd.readouterr().err
         expect = np.zeros(64, np.int32)
         expect[40] = 2
         assert np.array_equal(status, expect)
         keep = np.ones(len(back), bool)
         keep[tok_off[40]:tok_off[40] + 10] = False
         assert np.array_equal(back[keep], tokens[keep])
+
+
+def _set_split(monkeypatch, split):
+    """SC_HIP_DEC_SPLIT, or the default plan (None)."""
+    if split is None:
+        monkeypatch.delenv("SC_HIP_DEC_SPLIT", raising=False)
+    else:
+        monkeypatch.setenv("SC_HIP_DEC_SPLIT", split)
 
 
 def _random_chunks(codec, n, hi, seed):
@@ -923,21 +958,19 @@ def _random_chunks(codec, n, hi, seed):
 @pytest.mark.parametrize("n,seg", [(1, None), (3, 64), (33, None), (675, None), (675, 64), (675, 0), (1024, None),
                                    (1025, None), (2048, None)])
 def test_split_decode_matches_unsplit(codecs, capfd, monkeypatch, n, seg):
-    """Launches of at most 64 groups of 32 chunks decode split (workgroups
-    of a group share layer 0 and exchange its features every step): eight
-    workgroups per group up to 32 groups, four up to 64 (and four when
-    forced, SC_HIP_DEC_SPLIT=4).  One chunk, a partial group, two groups, 22
-    groups (the c1 case) over 256-step and 64-step segments and one launch,
-    32, 33 and 64 groups.  Tokens equal the input and the unsplit decode's
-    (SC_HIP_DEC_SPLIT=0)."""
+    """Launches of at most 64 groups of 32 chunks can decode split
+    (workgroups of a group share layer 0 and exchange its features every
+    step; SC_HIP_DEC_SPLIT): eight workgroups per group up to 32 groups, four
+    up to 64.  One chunk, a partial group, two groups, 22 groups (64 reads'
+    case) over 256-step and 64-step segments and one launch, 32, 33 and 64
+    groups.  Tokens equal the input, as the default (fed) decode's and the
+    unsplit one's (SC_HIP_DEC_SPLIT=0) do."""
     codec = codecs["lossless"]
     tokens, lengths, words, woff, wcnt = _random_chunks(codec, n, 700, n)
     _set_dec_env(monkeypatch, seg)
     groups = (n + 31) // 32
-    modes = [(None, "split launch p8" if groups <= 32 else "split launch p4")]
-    if groups <= 32:
-        modes.append(("4", "split launch p4"))
-    modes.append(("0", "launch"))
+    modes = [(None, "fed launch"), ("8", "split launch p8" if groups <= 32 else "launch"), ("4", "split launch p4"),
+             ("0", "launch")]
     for env, expect in modes:
         if env is None:
             monkeypatch.delenv("SC_HIP_DEC_SPLIT", raising=False)
@@ -976,12 +1009,14 @@ def test_ended_chunks_cost_a_split_group_nothing(codecs, monkeypatch):
     assert best[1] < 1.2 * best[0], best
 
 
-def test_split_decode_not_used_beyond_64_groups(codecs, capfd, monkeypatch):
+@pytest.mark.parametrize("split", ["4", "8"])
+def test_split_decode_not_used_beyond_64_groups(codecs, capfd, monkeypatch, split):
     """2,049 chunks make 65 groups, more than a split launch holds: one
     unsplit launch of 32-chunk workgroups."""
     codec = codecs["lossless"]
     tokens, lengths, words, woff, wcnt = _random_chunks(codec, 2049, 200, 3)
     _set_dec_env(monkeypatch, None)
+    monkeypatch.setenv("SC_HIP_DEC_SPLIT", split)
     capfd.readouterr()
     back, _ = codec.decompress_flat(words, woff, wcnt, lengths)
     log = capfd.readouterr().err
@@ -989,11 +1024,13 @@ def test_split_decode_not_used_beyond_64_groups(codecs, capfd, monkeypatch):
     assert np.array_equal(back, tokens)
 
 
+@pytest.mark.parametrize("split", ["8", "4", None])
 @pytest.mark.parametrize("lossy", [False, True])
-def test_split_decode_matches_oracle(codecs, oracle_mod, oracle_models, lossy):
-    """Split decode of 40 chunks (two groups, the second partial) with the
-    lossless and the lossy model: every chunk's tokens equal the oracle's
-    decode of the same words."""
+def test_split_decode_matches_oracle(codecs, oracle_mod, oracle_models, monkeypatch, lossy, split):
+    """Split decode (and the default, fed one) of 40 chunks (two groups, the
+    second partial) with the lossless and the lossy model: every chunk's
+    tokens equal the oracle's decode of the same words."""
+    _set_split(monkeypatch, split)
     name = "lossy" if lossy else "lossless"
     codec = codecs[name]
     tokens, lengths, words, woff, wcnt = _random_chunks(codec, 40, 300, 11 + lossy)
@@ -1005,9 +1042,12 @@ def test_split_decode_matches_oracle(codecs, oracle_mod, oracle_models, lossy):
         assert np.array_equal(back[tok_off[c]:tok_off[c] + lengths[c]], ref[c]), c
 
 
-def test_split_decode_corrupt_chunks(codecs, monkeypatch):
-    """Corrupt chunks in both groups of a split decode over 64-step
-    segments: each reports an invalid stream, every other chunk decodes."""
+@pytest.mark.parametrize("split", ["8", "4", None])
+def test_split_decode_corrupt_chunks(codecs, monkeypatch, split):
+    """Corrupt chunks in every group of a split decode over 64-step segments
+    and of a fed decode: each reports an invalid stream, every other chunk
+    decodes."""
+    _set_split(monkeypatch, split)
     codec = codecs["lossless"]
     tokens, lengths, words, woff, wcnt = _random_chunks(codec, 70, 400, 5)
     bad = [0, 33, 69]
@@ -1025,7 +1065,7 @@ def test_split_decode_corrupt_chunks(codecs, monkeypatch):
             assert np.array_equal(back[s], tokens[s]), i
 
 
-@pytest.mark.parametrize("split", ["0", None])
+@pytest.mark.parametrize("split", ["0", "8", None])
 def test_decode_of_garbage_and_damaged_chunks_matches_oracle(codecs, oracle_mod, oracle_models, monkeypatch, split):
     """Arbitrary words are a range-coded stream too: the decoder either
     reaches a quantile outside the table (an invalid stream) or returns
@@ -1033,11 +1073,11 @@ def test_decode_of_garbage_and_damaged_chunks_matches_oracle(codecs, oracle_mod,
     -- valid streams, 0 to 8 random words, and valid streams cut short or
     with one word changed -- plus five streams invalid at their first step,
     each chunk's status, and the tokens of every chunk that decodes, equal
-    the C oracle's; with the persistent decode
-    (split "0") and with the default plan, a split decode for this batch."""
+    the C oracle's; with the persistent decode (split "0"), the split one
+    ("8") and the default plan, a fed decode for this batch."""
     import ctypes
     codec = codecs["lossless"]
-    rng = np.random.default_rng(600 if split is None else 601)
+    rng = np.random.default_rng({None: 600, "0": 601, "8": 602}[split])
     n = 600
     lengths = rng.integers(1, 151, n).astype(np.int32)
     tokens = rng.integers(0, 60, int(lengths.sum())).astype(np.uint8)
@@ -1061,10 +1101,7 @@ def test_decode_of_garbage_and_damaged_chunks_matches_oracle(codecs, oracle_mod,
     off = np.zeros(n, np.int64)
     np.cumsum(cnt[:-1], dtype=np.int64, out=off[1:])
     flat = np.concatenate(streams + [np.zeros(1, np.uint32)])
-    if split is None:
-        monkeypatch.delenv("SC_HIP_DEC_SPLIT", raising=False)
-    else:
-        monkeypatch.setenv("SC_HIP_DEC_SPLIT", split)
+    _set_split(monkeypatch, split)
     back, status, tok_off = _decode_direct(codec, flat, off, cnt, lengths)
     # the oracle, every chunk's status (its Python wrapper raises on the first)
     om = oracle_models["lossless"]
@@ -1080,17 +1117,20 @@ def test_decode_of_garbage_and_damaged_chunks_matches_oracle(codecs, oracle_mod,
         assert np.array_equal(back[s], ref_tok[s]), i
 
 
-def test_split_decode_timeout_reports_status_and_redecodes_unsplit(codecs, monkeypatch):
+@pytest.mark.parametrize("split", ["8", "4", None])
+def test_split_decode_timeout_reports_status_and_redecodes_unsplit(codecs, monkeypatch, split):
     """With a spin limit of 0 polls (SC_HIP_DEC_SPIN=0; the default is
-    2**18) every wait of a split decode gives up at once: every chunk of
-    every group reports SC_STATUS_SYNC_TIMEOUT through the C ABI, also
-    through later step segments, and the kernels end normally.
+    2**18) every wait of a split decode, or of a fed one of up to 64 tiles,
+    gives up at once: every chunk of every group reports
+    SC_STATUS_SYNC_TIMEOUT through the C ABI, also through a split decode's
+    later step segments, and the kernels end normally.
     decompress_flat then decodes the timed-out chunks again with unsplit
     launches (SC_DEC_OPT_NO_SPLIT), which never wait, and returns the input;
     the next decode with the default limit is correct as well.  A corrupt
     chunk among them is still reported as such."""
     codec = codecs["lossless"]
     tokens, lengths, words, woff, wcnt = _random_chunks(codec, 40, 300, 9)
+    _set_split(monkeypatch, split)
     monkeypatch.setenv("SC_HIP_DEC_SPIN", "0")
     monkeypatch.setenv("SC_HIP_DEC_SEG", "64")
     _, status, _ = _decode_direct(codec, words, woff, wcnt, lengths)

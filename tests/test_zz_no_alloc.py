@@ -56,23 +56,33 @@ def _decode(codec, entry, words, woff, wcnt, lengths, host_lengths):
     return out.cpu().numpy()[:int(lengths.sum())], status.cpu().numpy()
 
 
+@pytest.mark.parametrize("split", ["0", None])
 @pytest.mark.parametrize("host_lengths", [True, False])
-def test_static_entry_matches_workspace_entry(codec, monkeypatch, host_lengths):
+def test_static_entry_matches_workspace_entry(codec, monkeypatch, capfd, host_lengths, split):
     """Call 1: 2 * 32 * n_cu + 150 chunks of up to 700 tokens (full-wave
     launches, leftover chunks paired into the last one's rows, three 256-step
     segments whose state goes through the static array); call 2, smaller:
-    900 chunks of up to 300 tokens (one launch of 32-chunk workgroups over
-    two segments).  The second call runs over the first call's leftover
-    state; both must equal the workspace entry point's output and the
-    original tokens."""
+    900 chunks of up to 300 tokens (SC_HIP_DEC_SPLIT=0: one launch of
+    32-chunk workgroups over two segments; by default one fed launch).  The
+    second call runs over the first call's leftover state; both must equal
+    the workspace entry point's output and the original tokens."""
     monkeypatch.delenv("SC_HIP_DEC_SEG", raising=False)
+    monkeypatch.setenv("SC_HIP_DEC_LOG", "1")
+    monkeypatch.setenv("SC_HIP_DEC_ROT", "0")
+    if split is None:
+        monkeypatch.delenv("SC_HIP_DEC_SPLIT", raising=False)
+    else:
+        monkeypatch.setenv("SC_HIP_DEC_SPLIT", split)
     n_cu = torch.cuda.get_device_properties(0).multi_processor_count
     for n, hi, seed in ((2 * 32 * n_cu + 150, 700, 1), (900, 300, 2)):
         tokens, lengths, words, woff, wcnt = _inputs(codec, n, 1, hi, seed)
         src = np.concatenate([[0], np.cumsum(lengths[:-1])]).astype(np.int64)   # input chunk starts
         order = np.argsort(-lengths, kind="stable")            # longest first, as decompress_flat
         s_len, s_woff, s_wcnt = lengths[order], woff[order], wcnt[order]
+        capfd.readouterr()
         ref_tok, ref_st = _decode(codec, "workspace", words, s_woff, s_wcnt, s_len, host_lengths)
+        log = capfd.readouterr().err
+        assert ("leftover 150 paired" if n > 900 else f"leftover 900 {'launch' if split else 'fed launch'}") in log, log
         got_tok, got_st = _decode(codec, "static", words, s_woff, s_wcnt, s_len, host_lengths)
         assert np.array_equal(got_st, ref_st) and not got_st.any()
         assert np.array_equal(got_tok, ref_tok)
@@ -93,8 +103,8 @@ def test_static_entry_rejects_more_chunks_than_its_array(codec):
 
 def test_static_entry_under_graph_capture(codec):
     """The entry point's callers include code under HIP graph capture: 40
-    chunks over two 256-step segments (a batch that decodes split when not
-    captured; a capturing stream gets the unsplit launches) captured once
+    chunks over two or three 256-step segments (a batch that decodes fed when
+    not captured; a capturing stream gets the unsplit launches) captured once
     and replayed three times, with eager work between the replays that
     overwrites the outputs; every replay equals the eager decode and the
     input."""
