@@ -333,10 +333,11 @@ __device__ __forceinline__ void fed_feeder(const ModelDev &M, uint8_t *s_mem, co
         int tn[FED_POS];
         v4u part[WAVES];
         // (a reduction that finish() has done is repeated without its
-        // barrier and stored nowhere)
+        // barrier and stored nowhere: no records, and no scalar offset, which
+        // the range check subtracts from their number)
         const __amdgpu_buffer_rsrc_t rs_open = fed_sums(xch, __builtin_amdgcn_readfirstlane(ptile),
                                                         __builtin_amdgcn_readfirstlane(open ? FED_SUMS : 0));
-        const int off_open = __builtin_amdgcn_readfirstlane(poff);
+        const int off_open = __builtin_amdgcn_readfirstlane(open ? poff : 0);
         __builtin_amdgcn_sched_barrier(0);
         // One position per region: its products, the next position's operand
         // reads, the next item's address of this position, and a piece of
