@@ -55,6 +55,69 @@ def test_round_trip_and_corrupt_chunk(arch, oracle_mod):
         codec.decompress_chunks(enc, lengths)
 
 
+@pytest.mark.parametrize("fused", ["0", "1"])
+def test_requantisation_beyond_32_bit_products(oracle_mod, monkeypatch, fused):
+    """Layers whose constants need the whole 64-bit product (a shift below 32,
+    or a multiplier of 2**31 that becomes 2**30 with a shift of 31) beside
+    ones that do not; one output of such a layer takes the whole layer there."""
+    import dataclasses
+    from sigcomp_amd.model_io import make_layer, random_int_model
+    from sigcomp_amd.quant_mlp_export import QuantMLPCompression
+    monkeypatch.setenv("SC_HIP_GEN_FUSED", fused)
+    rng = np.random.default_rng(31)
+    m = random_int_model(seed=31, window=7, emb_dim=32, hidden=96, n_hidden=4, per_channel=True)
+    layers = list(m.layers)
+
+    def change(i, outputs, m0, shift):
+        L = layers[i]
+        new_m0, new_shift = np.array(L.m0, np.int64), np.array(L.shift, np.int32)
+        new_m0[outputs], new_shift[outputs] = m0(new_m0[outputs], new_shift[outputs]), shift
+        layers[i] = make_layer(L.weight, L.bias, new_m0, new_shift, L.relu)
+
+    scaled = lambda to: lambda m0, sh: np.maximum(m0 >> (sh - to), 1)   # the same factor at another shift
+    change(0, slice(None), scaled(31), 31)
+    change(1, slice(5, 6), scaled(24), 24)
+    change(2, slice(0, 96, 7), lambda m0, sh: 1 << 31, 32)
+    change(2, slice(1, 96, 7), lambda m0, sh: 1 << 31, 40)
+    change(4, slice(3, 200), scaled(30), 30)
+    m = dataclasses.replace(m, layers=layers)
+    codec = QuantMLPCompression(chunk_len=300, gpu=0, model=m)
+    om = oracle_mod.OracleModel(m)
+    ctx = rng.integers(0, 257, (100, m.window)).astype(np.int64)
+    ref = oracle_mod.mlp_forward(om, ctx)
+    assert len(np.unique(ref)) > 30   # (not saturated throughout)
+    assert np.array_equal(codec.hip.forward_windows(torch.from_numpy(ctx).cuda(), "logits").cpu().numpy(), ref)
+    lengths = [1, 64, 129]
+    chunks = [rng.integers(0, 60, n).astype(np.uint8) for n in lengths]
+    enc = codec.compress_chunks(chunks)
+    assert enc == oracle_mod.compress_chunks(om, chunks)
+    assert all(np.array_equal(a, b) for a, b in zip(chunks, codec.decompress_chunks(enc, lengths)))
+
+
+def test_more_tiles_than_cus(oracle_mod, monkeypatch):
+    """A workgroup that takes several 32-row tiles: forward of more than 32
+    rows per CU, compress of more 32-step tiles than CUs (some of them past
+    their chunk's end)."""
+    from sigcomp_amd.model_io import random_int_model
+    from sigcomp_amd.quant_mlp_export import QuantMLPCompression
+    monkeypatch.setenv("SC_HIP_GEN_FUSED", "1")
+    n_cu = torch.cuda.get_device_properties(0).multi_processor_count
+    m = random_int_model(seed=4, window=9, emb_dim=16, hidden=48, n_hidden=2, per_channel=True)
+    codec, om = QuantMLPCompression(chunk_len=300, gpu=0, model=m), oracle_mod.OracleModel(m)
+    rng = np.random.default_rng(6)
+    ctx = rng.integers(0, 257, (2 * 32 * n_cu + 70, m.window)).astype(np.int64)
+    ref = oracle_mod.mlp_forward(om, ctx)
+    dev = torch.from_numpy(ctx).cuda()
+    assert np.array_equal(codec.hip.forward_windows(dev, "logits").cpu().numpy(), ref)
+    assert np.array_equal(codec.hip.forward_windows(dev, "cdf").cpu().numpy().astype(np.int64),
+                          oracle_mod.logits_to_cdf(ref, m.exp_lut))
+    lengths = rng.choice([0, 1, 31, 32, 33, 64, 100, 128, 129, 300], 2 * n_cu + 11)
+    chunks = [rng.integers(0, 60, n).astype(np.uint8) for n in lengths]
+    enc = codec.compress_chunks(chunks)
+    assert enc == oracle_mod.compress_chunks(om, chunks)
+    assert all(np.array_equal(a, b) for a, b in zip(chunks, codec.decompress_chunks(enc, list(lengths))))
+
+
 def _wide():
     from sigcomp_amd.model_io import random_int_model
     from sigcomp_amd.quant_mlp_export import QuantMLPCompression
