@@ -352,7 +352,6 @@ __device__ __forceinline__ void fed_feeder(const ModelDev &M, uint8_t *s_mem, co
             if constexpr (i > 0) {
                 ea[i - 1] = emb_off(sn + p0 + i - 1 < WIN ? SOS : tn[i - 1], 0) + kg;
                 asm volatile("" : "+v"(ea[i - 1]));   // here, not after the last product
-
             }
             if constexpr (i < 4) red_put(i);
             if constexpr (i == RED_READ) {
@@ -608,7 +607,7 @@ __device__ __forceinline__ void fed_head(const ModelDev &M, uint8_t *s_mem, cons
             for (int x = 0; x < PPD; ++x)
 #pragma unroll
                 for (int j = 0; j < PNT; ++j) w[0][x][j] = wload_s(rs1, voff, ((nb0 + j) * KTH + x) * 1024);
-            // layer 0: both halves' sums plus the newest token's position
+            // layer 0: the feeders' sums plus the newest token's position
 #pragma unroll
             for (int i = 0; i < RT; ++i) {
                 const int ea = (int)c.last[i * 32 + rl] + kg;
@@ -645,7 +644,7 @@ __device__ __forceinline__ void fed_head(const ModelDev &M, uint8_t *s_mem, cons
             pipe_hidden<RT, false, UNI>(M.layer[l - 1], M.layer[l], M.layer[l + 1], s_act, s_parw, l, accA, accB, w,
                                         pk, wave, lane);
         load_flags();   // read back behind the last hidden layer
-        pipe_hidden<RT, false, UNI, false, false, !RES>(M.layer[last - 2], M.layer[last - 1], M.layer[last], s_act,
+        pipe_hidden<RT, false, UNI, false, !RES>(M.layer[last - 2], M.layer[last - 1], M.layer[last], s_act,
                                                         s_parw, last - 1, accA, accB, w, pk, wave, lane);
         if constexpr (RES) {
             // the next step's sums travel beside the output layer, which

@@ -399,7 +399,8 @@ __device__ __forceinline__ void gen_mlp_rows(const ModelDev &M, const GenLds &P,
                     for (int s = 0; s < GEN_BLK; ++s) {
                         // 16 columns of one position (E is a multiple of 16);
                         // columns past the window have zero weights
-                        // (exact: fewer than 2**12 chunks, 2**20 > 2**12 * chunks per position)
+                        // (exact while ch * (E / 16) < 2**20: the windows and widths
+                        // that fit the LDS reach 174,000)
                         const int ch = (kt0 + s) * 2 + g, p = min((int)(((uint32_t)ch * P.inv) >> 20), W - 1);
                         addr[s] = (int)s_ctx[slot(p) * 32 + rl] * P.emb_stride + min(ch * 16 - p * E, E - 16);
                     }

@@ -377,18 +377,15 @@ __device__ __forceinline__ void pipe_schedule() {
 // layer's first k-steps.  Both passes' GEMMs start from their bias tiles.
 // FRESH: the whole previous layer is already in regions A and B (visible),
 // accB holds nothing to requantise (the first layer after a layer 0 whose
-// features were gathered from several workgroups).  PRE: w[1] holds the
-// layer's k-steps PPD .. 2 PPD - 1 as well at entry (2 PPD = 16: all of pass
-// 0).  NEXTW = false: no weights of the next layer are loaded (w[0] holds
-// nothing at exit).
-template <int RT, bool LASTL, bool UNI, bool FRESH = false, bool PRE = false, bool NEXTW = true>
+// features were gathered from several workgroups).  NEXTW = false: no
+// weights of the next layer are loaded (w[0] holds nothing at exit).
+template <int RT, bool LASTL, bool UNI, bool FRESH = false, bool NEXTW = true>
 __device__ __forceinline__ void pipe_hidden(const LayerDev &Lp, const LayerDev &L, const LayerDev &Ln, uint8_t *s_act,
                                             uint32_t *s_parw, int l, v16i (&accA)[PNT][RT],
                                             v16i (&accB)[PNT][RT], v4i (&w)[2][ppd<RT>()][PNT],
                                             uint32_t (&pk)[PNT][RT][4], int wave, int lane) {
     constexpr int PPD = ppd<RT>();
     constexpr int NV = LASTL ? KTH : 2 * KTH;
-    static_assert(!PRE || (2 * PPD == KTH && !LASTL), "PRE holds pass 0 of a hidden layer");
     constexpr int MF = PNT * RT;
     const int g = lane >> 5, voff = lane * 16;
     const int bbase = pact_off(lane & 31, g);
@@ -424,16 +421,14 @@ __device__ __forceinline__ void pipe_hidden(const LayerDev &Lp, const LayerDev &
         // ago; the 2 * LANE parameter loads at the top of this function
         // are younger than the first PPD steps' fragments) and its B
         // fragments, instead of the compiler's wait before each first use
-        // (PRE: the first 2 PPD steps' fragments were all issued before the
-        // parameter loads; without NEXTW the last PPD steps issue none)
-        constexpr int ahead = PRE && v < PPD ? (2 * PPD - 1 - v) * PNT : !NEXTW && v > NV - PPD ? (NV - 1 - v) * PNT : (PPD - 1) * PNT;
-        wait_counts<ahead + ((v < PPD || (PRE && v < 2 * PPD)) && !LASTL ? 2 * Slot<UNI>::LANE : 0), 0>();
+        // (without NEXTW the last PPD steps issue none)
+        constexpr int ahead = !NEXTW && v > NV - PPD ? (NV - 1 - v) * PNT : (PPD - 1) * PNT;
+        wait_counts<ahead + (v < PPD && !LASTL ? 2 * Slot<UNI>::LANE : 0), 0>();
         // next step's B fragments (none across a barrier)
         if constexpr (v != 7 && v != NV - 1) read_b<RT>(s_act, bbase, (kt + 1) % KTH, b[(kt + 1) & 1]);
         // weights PPD steps ahead: this layer, else the next layer's pass 0
         constexpr int vp = v + PPD;
-        if constexpr (PRE && vp < 2 * PPD) {
-        } else if constexpr (vp < NV) {
+        if constexpr (vp < NV) {
             constexpr int pp_ = vp / KTH, kp = vp % KTH;
 #pragma unroll
             for (int j = 0; j < PNT; ++j)
@@ -478,7 +473,7 @@ __device__ __forceinline__ void pipe_hidden(const LayerDev &Lp, const LayerDev &
             for (int i = 0; i < RT; ++i)
                 acc[j][i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(w[set][slot][j], b[kt & 1][i],
                                                                   kt == 0 ? bias[j] : acc[j][i], 0, 0, 0);
-        constexpr int VM = (PRE && vp < 2 * PPD) || (!NEXTW && vp >= NV) ? 0 : PNT;
+        constexpr int VM = !NEXTW && vp >= NV ? 0 : PNT;
         pipe_schedule<MF, (v != 7 && v != NV - 1 ? RT : 0) + (UNI ? 0 : 3) + (v == KTH - 1 ? 4 * PNT : 0), VM, VA>();
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (v == 7) {
