@@ -62,6 +62,10 @@ def _on(t, device, dtype) -> torch.Tensor:
 
 
 def _lut_on(exp_lut, device) -> torch.Tensor:
+    # (as_tensor straight to int64: a list of floats would pass through
+    # float32, which does not hold the larger entries)
+    if not isinstance(exp_lut, torch.Tensor):
+        exp_lut = torch.as_tensor(exp_lut, dtype=torch.int64)
     lut = _on(exp_lut, device, torch.int64)
     if lut.shape != (VOCAB_SIZE,):
         raise ValueError("exp_lut must have shape (256,)")
