@@ -124,10 +124,10 @@ int sc_mlp_forward_cdf(const sc_model *model, const int64_t *ctx, int64_t rows, 
 
 /* sc_mlp_forward (logits non-null) or sc_mlp_forward_cdf (cdf non-null;
  * exactly one of them) with device workspace: with at least
- * sc_mlp_forward_workspace_bytes(rows) bytes, calls of few rows run in two
- * launches, layer 0 spread over the device and then the rest (the same
- * results); with less, and for calls that this does not help (0 bytes), as
- * without workspace.  Replaces GPUBitExactMLPDecoder._ar_step
+ * sc_mlp_forward_workspace_bytes(rows) bytes, 16-byte aligned, calls of few
+ * rows run in two launches, layer 0 spread over the device and then the rest
+ * (the same results); with less or otherwise aligned, and for calls that this
+ * does not help (0 bytes), as without workspace.  Replaces GPUBitExactMLPDecoder._ar_step
  * (quant_mlp_export.py:133-138) as those do. */
 int64_t sc_mlp_forward_workspace_bytes(int64_t rows);
 int sc_mlp_forward_ws(const sc_model *model, const int64_t *ctx, int64_t rows, int8_t *logits, int32_t *cdf,

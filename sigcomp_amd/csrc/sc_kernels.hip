@@ -1048,7 +1048,8 @@ int sc_mlp_forward_ws(const sc_model *m, const int64_t *ctx, int64_t rows, int8_
     if (rows == 0) return SC_OK;
     if ((!logits) == (!cdf)) return fail(SC_ERR_ARG, "exactly one of logits and cdf");
     const int64_t need = sc_mlp_forward_workspace_bytes(rows);
-    if (need == 0 || !workspace || workspace_bytes < need || !ctx ||
+    // (the features are read and written 16 bytes at a time)
+    if (need == 0 || !workspace || (uintptr_t)workspace % 16 || workspace_bytes < need || !ctx ||
         (m->dev.pipe != CORE_PIPE_UNI && m->dev.pipe != CORE_PIPE))
         return mlp_context_launch(m, ctx, rows, logits, cdf, status, stream, logits ? OUT_LOGITS : OUT_CDF32);
     DeviceGuard guard(m->device);

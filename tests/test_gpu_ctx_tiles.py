@@ -41,7 +41,7 @@ def test_tile_sizes(codec, oracle_mod, rows):
     ref = oracle_mod.mlp_forward(oracle_mod.OracleModel(m), ctx[pick])
     assert np.array_equal(logits[pick], ref)
     assert np.array_equal(cdf[pick].astype(np.int64), oracle_mod.logits_to_cdf(ref, m.exp_lut))
-    # every row, through calls of another tile size
+    # every row, through calls of another tile size (the same one up to 5,000 rows)
     again = np.concatenate([c.hip.forward_windows(dev[i:i + 5000], "logits").cpu().numpy() for i in range(0, rows, 5000)])
     assert np.array_equal(again, logits)
 
@@ -56,3 +56,25 @@ def test_no_rows_and_bad_token(codec):
         ctx[69, 63] = bad
         with pytest.raises(ValueError):
             c.hip.forward_windows(ctx, "logits")
+
+
+@pytest.mark.parametrize("rows", [1, 33, 4096])
+def test_workspace_that_is_not_used(codec, rows):
+    """Without workspace, with too little and with one that is not 16-byte
+    aligned: one launch, the workspace untouched, the same results."""
+    from sigcomp_amd import _hip
+    m, c = codec
+    ctx = torch.from_numpy(np.random.default_rng(rows).integers(0, 257, (rows, 64)).astype(np.int64)).cuda()
+    want = {k: c.hip.forward_windows(ctx, k) for k in ("logits", "cdf")}
+    need = _hip.lib().sc_mlp_forward_workspace_bytes(rows)
+    ws = torch.full((need + 16,), 0xAB, dtype=torch.uint8, device="cuda")
+    assert need > 0 and ws.data_ptr() % 16 == 0
+    for ptr, nbytes in ((None, 0), (ws.data_ptr(), need - 1), (ws.data_ptr() + 1, need), (ws.data_ptr() + 8, need)):
+        for out in ("logits", "cdf"):
+            got, status = torch.zeros_like(want[out]), torch.zeros(1, dtype=torch.int32, device="cuda")
+            to = (got.data_ptr(), None) if out == "logits" else (None, got.data_ptr())
+            _hip.check(_hip.lib().sc_mlp_forward_ws(c.hip.handle, ctx.data_ptr(), rows, *to, status.data_ptr(), ptr, nbytes,
+                                                    _hip.stream_ptr()))
+            torch.cuda.synchronize()
+            assert torch.equal(got, want[out]) and not status.item()
+        assert (ws == 0xAB).all()
