@@ -1298,17 +1298,25 @@ struct RotPlan {
 // A launch's time beyond its steps (tables staged, the first layer 0 and the
 // last epilogue alone, the workgroups' drift), in DEC_STEP_COST's unit.
 constexpr int64_t DEC_LAUNCH_COST = 400;
+// The step costs are those of a device full of whole chunks.  Where most
+// chunks end early, steps of full waves get cheaper with the workgroups that
+// have ended, while rotating launches stay full: 20,480 chunks of geometric
+// lengths about 200, at most 1,024, take 65.7 ms as full waves (78 by the
+// costs) and 67.7 rotating (72); 25,000 of them 87.8 and 74.8 (109 and 80).
+constexpr double ROT_MARGIN_ENDED = 0.15;
 
 static RotPlan rot_plan(const int32_t *len, int64_t n, int64_t cu) {
     RotPlan best;
+    std::vector<int32_t> from((size_t)((n + 31) / 32));   // longest chunk of 32 and all after them
+    for (int64_t i = (int64_t)from.size() - 1, m = 0; i >= 0; --i) {
+        m = std::max<int64_t>(m, *std::max_element(len + i * 32, len + std::min(n, i * 32 + 32)));
+        from[(size_t)i] = (int32_t)m;
+    }
     for (int rt = 1; rt <= RT_TILE; ++rt) {
         const int64_t R = 32 * rt, G = (n + R - 1) / R;
         if (G <= cu / 2) continue;
-        std::vector<int32_t> longest((size_t)G, 0);   // of the group and all after it
-        for (int64_t i = n - 1, m = 0; i >= 0; --i) {
-            m = std::max<int64_t>(m, len[i]);
-            longest[(size_t)(i / R)] = (int32_t)m;
-        }
+        std::vector<int32_t> longest((size_t)G);   // of the group and all after it
+        for (int64_t i = 0; i < G; ++i) longest[(size_t)i] = from[(size_t)(i * rt)];
         for (int64_t seg = DEC_SEG_STEPS; seg >= WIN; seg /= 2) {
             const int64_t K = std::max<int64_t>(1, (longest[0] + seg - 1) / seg);
             // groups with steps in segment k (k does not fall from call to call)
@@ -1466,8 +1474,10 @@ static int decompress_run(const sc_model *m, const uint32_t *words, const int64_
     const int64_t maxlen = std::max(len_max, pair ? pair_max : 0);
     // The plan's cost against rotating launches': its launches' longest
     // chunks' steps, the pairs' or the leftover launch's.  Rotating launches
-    // have to be 2% cheaper, which is what the step costs are good to.  (They
-    // need the lengths here, so a call without lengths_host keeps the plan.)
+    // have to be 2% cheaper, which is what the step costs are good to, and
+    // more the shorter the chunks are against the longest (ROT_MARGIN_ENDED).
+    // (They need the lengths here, so a call without lengths_host keeps the
+    // plan.)
     RotPlan rot;
     const char *rot_env = getenv("SC_HIP_DEC_ROT");   // "0": never rotate (comparisons)
     // (Chunks beyond 2**20 tokens keep the plan too: the host lists every launch.)
@@ -1482,7 +1492,10 @@ static int decompress_run(const sc_model *m, const uint32_t *words, const int64_
             at = end;
         }
         rot = rot_plan(lengths_host, n_chunks, cu);
-        if (rot.cost > cost / 50 * 49) rot.rt = 0;
+        int64_t sum = 0;
+        for (int64_t i = 0; i < n_chunks; ++i) sum += std::max(lengths_host[i], 0);
+        const double ended = len_max > 0 ? 1 - (double)sum / ((double)n_chunks * len_max) : 0;
+        if ((double)rot.cost > (double)cost * (0.98 - ROT_MARGIN_ENDED * ended)) rot.rt = 0;
     }
     if (const char *log = getenv("SC_HIP_DEC_LOG"); log && std::strcmp(log, "1") == 0) {   // what is launched
         if (rot.rt) {

@@ -124,3 +124,23 @@ def test_rotating_decode_under_graph_capture(codec, monkeypatch, capfd):
         graph.replay()
         got, status = call.results()
         assert not status.any() and np.array_equal(got, tokens), rep
+
+
+@pytest.mark.parametrize("n,rotates", [(20480, False), (25000, True)])
+def test_batches_of_mostly_short_chunks(codec, monkeypatch, capfd, n, rotates):
+    """Full waves whose workgroups end early take less than their longest
+    chunks' steps, so that rotating launches have to promise more: 65.7 ms as
+    full waves and 67.7 rotating for the first of these, 87.8 and 74.8 for
+    the second."""
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the chunk counts are for 256 CUs")
+    rng = np.random.default_rng(n)
+    lengths = -np.sort(-np.minimum(rng.geometric(1 / 200, n), 1024)).astype(np.int32)
+    lengths[0] = 1024
+    tokens = rng.integers(0, 60, int(lengths.sum())).astype(np.uint8)
+    words, woff, wcnt = (np.array(a) for a in codec.compress_flat(tokens, lengths))
+    monkeypatch.setenv("SC_HIP_DEC_LOG", "1")
+    capfd.readouterr()
+    back, _ = codec.decompress_flat(words, woff, wcnt, lengths)
+    assert ("rotating" in capfd.readouterr().err) == rotates
+    assert np.array_equal(back, tokens)
