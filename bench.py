@@ -39,8 +39,10 @@ import argparse
 import glob
 import json
 import os
+import re
 import subprocess
 import sys
+import tempfile
 import threading
 import time
 from pathlib import Path
@@ -187,24 +189,48 @@ def roofline(kernel, tokens, seconds, config, direction):
 PEAK_L1_GBS_PER_CU = 64 * 2.4   # vector L1 fill: 64 bytes per clock at the 2.4 GHz peak engine clock
 
 
-def split_roofline(model, lengths, seconds, n_cu):
-    """Bound of a decode that runs split (fewer than 32 x n_cu chunks in at
-    most 64 groups of 32 that the CUs hold with 4 or 8 workgroups each, as
-    sc_decompress_chunks plans it): each active CU streams its share of
-    layer 0 plus every later layer's weights through its vector L1 once per
-    step.  None when the decode does not run split."""
-    n = len(lengths)
-    groups = -(-n // 32)
-    if n >= 32 * n_cu or groups > 64 or groups * 4 > n_cu:
-        return None
-    p = 8 if groups * 8 <= n_cu else 4
-    per_cu = model.layers[0].n * model.layers[0].k // p + sum(L.n * L.k for L in model.layers[1:])
-    steps = int(lengths.max())
+def decode_log(decompress):
+    """The line sc_decompress_chunks writes about the launches of one call
+    (SC_HIP_DEC_LOG=1, standard error)."""
+    with tempfile.TemporaryFile() as f:
+        sys.stderr.flush()
+        keep = os.dup(2)
+        os.environ["SC_HIP_DEC_LOG"] = "1"
+        os.dup2(f.fileno(), 2)
+        try:
+            decompress()
+        finally:
+            os.dup2(keep, 2)
+            os.close(keep)
+            del os.environ["SC_HIP_DEC_LOG"]
+        f.seek(0)
+        return f.read().decode().strip().partition(": ")[2]
+
+
+def small_decode_roofline(model, launches, n, steps, seconds):
+    """Bound of a decode of n chunks that runs as one fed or split launch
+    (`launches`: its log): the weights that a workgroup on a chunk's chain
+    streams through its CU's vector L1 once per step.  A fed head streams the
+    hidden layers, and the output layer if it has 64 rows (32 rows keep it in
+    registers; layer 0 lies in the feeders' registers); a split workgroup its
+    share of layer 0 and every later layer.  None for any other decode."""
+    size = [L.n * L.k for L in model.layers]
+    if m := re.search(rf"leftover {n} fed launch .* fed (\d+)\+(\d+)x(\d+) rt (\d)", launches):
+        heads, sets, slices, rt = map(int, m.groups())
+        kernel, key = f"k_decompress_fed<{rt}>", "roofline_fed"
+        per_cu = sum(size[1:-1]) + (size[-1] if rt > 1 else 0)
+        active = f"{heads} heads of {32 * rt} chunks and {sets * slices} feeders"
+    elif m := re.search(rf"leftover {n} split launch p(\d)", launches):
+        p = int(m.group(1))
+        kernel, key = f"k_decompress (split, {p} workgroups per 32-chunk group)", "roofline_split"
+        per_cu = size[0] // p + sum(size[1:])
+        active = f"{-(-n // 32) * p} CUs"
+    else:
+        return {}
     gbs = per_cu * steps / seconds / 1e9
-    return {"kernel": f"k_decompress (split, {p} workgroups per 32-chunk group)", "bound": "vector L1 fill per CU",
-            "achieved": round(gbs, 2), "peak": PEAK_L1_GBS_PER_CU, "unit": "GB/s per CU",
-            "frac": round(gbs / PEAK_L1_GBS_PER_CU, 4),
-            "algorithmic": f"{per_cu} weight bytes per CU per step x {steps} steps, {groups * p} CUs active"}
+    return {key: {"kernel": kernel, "bound": "vector L1 fill per CU", "achieved": round(gbs, 2),
+                  "peak": PEAK_L1_GBS_PER_CU, "unit": "GB/s per CU", "frac": round(gbs / PEAK_L1_GBS_PER_CU, 4),
+                  "algorithmic": f"{per_cu} weight bytes per CU of the chain per step x {steps} steps; {active}"}}
 
 
 def calibration_copy(dev, copy_mib):
@@ -269,10 +295,18 @@ def run_codec(name, steps, warmup, sampler, n_reads=None, e2e=True, copy_mib=0):
                                           _hip.ptr(dstatus), o_len_host.ctypes.data, _hip.ptr(dws),
                                           dws.numel(), stream.cuda_stream))
 
+    launches = []   # the first decode's log
+
+    def decompress_noted():
+        if launches:
+            decompress()
+        else:
+            launches.append(decode_log(decompress))
+
     calibration_copy(dev, copy_mib)
     with torch.cuda.device(dev), torch.cuda.stream(stream):
         for w in range(warmup):
-            compress(); decompress()
+            compress(); decompress_noted()
             stream.synchronize()
         log(f"[bench] {name}: {warmup} warmup steps done")
         ev = [[torch.cuda.Event(enable_timing=True) for _ in range(3)] for _ in range(steps)]
@@ -282,7 +316,7 @@ def run_codec(name, steps, warmup, sampler, n_reads=None, e2e=True, copy_mib=0):
             ev[k][0].record(stream)
             compress()
             ev[k][1].record(stream)
-            decompress()
+            decompress_noted()
             ev[k][2].record(stream)
         stream.synchronize()
         torch.cuda.synchronize()
@@ -313,12 +347,12 @@ def run_codec(name, steps, warmup, sampler, n_reads=None, e2e=True, copy_mib=0):
         "parity": {"round_trip_all_chunks": True, "oracle_sample_chunks": parity},
         "wall_s_timed": round(wall, 3),
         "power": power_fields(sampler.window(t0, t1), t_c + t_d, samples),
-        "roofline": roofline("k_decompress", n_tokens, t_d, name, "decoded"),
+        "decode_launches": launches[0],
+        "roofline": roofline("k_decompress_fed" if f"leftover {n} fed launch" in launches[0] else "k_decompress",
+                             n_tokens, t_d, name, "decoded"),
         "roofline_compress": roofline("k_compress_mlp", n_tokens, t_c, name, "coded"),
+        **small_decode_roofline(codec.model, launches[0], n, int(lengths.max()), t_d),
     }
-    rl1 = split_roofline(codec.model, lengths, t_d, torch.cuda.get_device_properties(0).multi_processor_count)
-    if rl1:
-        res["roofline_split"] = rl1
     if e2e:
         # the first pass also allocates the pinned staging buffers (torch keeps
         # them cached): report the second, as a process that compresses
