@@ -274,7 +274,7 @@ int sc_decompress_chunks(const sc_model *model, const uint32_t *words, const int
 /* sc_decompress_chunks with options (a bitwise or of SC_DEC_OPT_*; any other
  * bit is SC_ERR_ARG).  SC_DEC_OPT_NO_SPLIT: every launch runs unsplit (one
  * workgroup per 32-chunk tile, no wait between workgroups), as
- * QuantMLPCompression.decompress_flat re-runs the chunks of a split launch
+ * QuantMLPCompression.decompress_flat re-runs the chunks of a fed or split launch
  * that reported SC_STATUS_SYNC_TIMEOUT.  Replaces the same reference call
  * as sc_decompress_chunks (quant_mlp_export.py:325-377). */
 #define SC_DEC_OPT_NO_SPLIT 1

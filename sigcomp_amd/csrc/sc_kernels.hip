@@ -776,7 +776,7 @@ constexpr int DEC_SEG_STEPS = 256;
 // Decode state of sc_decompress_chunks_static: a file-scope device array
 // (each GPU the library runs on holds its own copy until the process ends)
 // with the coder state of up to SC_STATIC_DEC_MAX_CHUNKS chunks, then the
-// launch plan's four length statistics, then the split decode's exchange
+// launch plan's four length statistics, then the fed or split decode's exchange
 // buffers and flags for XCH_MAX_GROUPS groups.  Host code never passes `scratch`
 // itself (in host code the name is a stand-in, not a device address): the
 // address of the current device's copy comes from hipGetSymbolAddress.
@@ -1438,13 +1438,13 @@ static int decompress_run(const sc_model *m, const uint32_t *words, const int64_
     // pair exceeds its longest chunk; the rt = 1 launch costs the longest
     // leftover chunk's steps
     // the launch of rt = 1 workgroups that takes what the full waves leave
-    // runs split when its 32-chunk groups fit: 8 workgroups per group when
-    // the CUs hold them, else 4 (SC_HIP_DEC_SPLIT=0: never, 4 or 8: only
-    // that split, for comparisons)
+    // runs fed (below), or split when that has no room and its 32-chunk
+    // groups fit: 8 workgroups per group when the CUs hold them, else 4
+    // (SC_HIP_DEC_SPLIT=0: neither, 4 or 8: only that split, for comparisons)
     const char *split_env = getenv("SC_HIP_DEC_SPLIT");
     const int split_force = split_env ? atoi(split_env) : -1;
-    // (a stream under graph capture gets the unsplit launches: the split
-    // one is a cooperative launch)
+    // (a stream under graph capture gets the unsplit launches: the fed and
+    // split ones are cooperative launches)
     const bool split_ok = m->dev.pipe == CORE_PIPE_UNI && xch && split_force != 0 &&
                           !(options & SC_DEC_OPT_NO_SPLIT) && capture == hipStreamCaptureStatusNone;
     // polls before a wait for the peers gives up (SC_HIP_DEC_SPIN: a lower
@@ -1674,7 +1674,7 @@ int sc_decompress_chunks_static(const sc_model *m, const uint32_t *words, const 
     void *base = scratch_ptr(m->device, &rc);
     if (!base) return rc;
     // every DecState is written by a segment before a later one reads it and
-    // the statistics are written before they are read; a split launch clears
+    // the statistics are written before they are read; a fed or split launch clears
     // its step flags itself (a kernel, no memset)
     DecState *state = (DecState *)base;
     int32_t *stat_dev = (int32_t *)((char *)base + SCRATCH_STATE_BYTES);

@@ -453,7 +453,7 @@ class QuantMLPCompression(ReadFramingMixin):
             st = h_status.numpy()
             late = np.flatnonzero(st == _hip.SC_STATUS_SYNC_TIMEOUT)
             if len(late):
-                # a split launch whose workgroups timed out waiting for each
+                # a fed or split launch whose workgroups timed out waiting for each
                 # other (one of them was not scheduled in time): its chunks
                 # are decoded again, each an independent stream, by unsplit
                 # launches that never wait between workgroups
