@@ -932,7 +932,8 @@ def run_all(args):
                    "compress_ms": c3["compress_ms"], "roofline": c3["roofline_compress"],
                    "note": "the headline's compress half"},
             "c4": {**{k: c3[k] for k in keep}, "decompress_msamples_s": c3["decompress_msamples_s"],
-                   "decompress_ms": c3["decompress_ms"], "roofline": c3["roofline"],
+                   "decompress_ms": c3["decompress_ms"], "decode_launches": c3["decode_launches"],
+                   "roofline": c3["roofline"],
                    "note": "the headline's decompress half (the c3 archive's streams)"},
             "c5": c5,
         }

@@ -1215,6 +1215,12 @@ constexpr int FED_RT_MAX = 2;
 // feeders (2,048-token chunks, lossless model).
 constexpr int FED_HEAD_COST[FED_RT_MAX + 1] = {0, 202, 310}, FED_TEN_TILES_COST = 174;
 constexpr int64_t FED_SET_AIM = 6;   // tiles per feeder set while CUs are free
+// What a fed and a split launch take beyond their steps and an unsplit
+// launch's start (the feeders' weights and tables, the flags' clearing, the
+// second launch of more than 64 tiles): decodes of one to three steps are
+// cheaper without (8,191 chunks of 1 token: fed 133 us, unsplit 88; of 6: 376
+// and 385; 700 chunks of 1: fed 77, split 70; of 3: 115 and 121).
+constexpr int FED_SETUP_COST = 290, FED_SETUP_COST_RETRY = 140, SPLIT_SETUP_COST = 160;
 
 // The cheapest fed launch of n chunks on `cu` CUs with xch_cap bytes of
 // exchange memory: a head's chain or its set's feeders, whichever takes
@@ -1276,6 +1282,19 @@ static void host_len_stats(const int32_t *len, int64_t n, int64_t g0, int64_t G,
     }
 }
 
+static int32_t longest_of(const int32_t *len, int64_t n) {
+    int32_t m = 0;
+    for (int64_t i = 0; i < n; ++i) m = std::max(m, len[i]);
+    return m;
+}
+// The longest chunk of every 32.
+static std::vector<int32_t> longest_of_32(const int32_t *len, int64_t n) {
+    std::vector<int32_t> m((size_t)((n + 31) / 32));
+    for (int64_t i = 0; i < (int64_t)m.size(); ++i)
+        m[(size_t)i] = longest_of(len + i * 32, std::min<int64_t>(n - i * 32, 32));
+    return m;
+}
+
 // Rotating decode launches.  A chunk's steps are serial, but its coder state
 // lies in memory between step segments, so the workgroups of a launch need
 // not be those of the last one: where the chunks are no whole number of full
@@ -1305,15 +1324,12 @@ constexpr int64_t DEC_LAUNCH_COST = 400;
 // costs) and 67.7 rotating (72); 25,000 of them 87.8 and 74.8 (109 and 80).
 constexpr double ROT_MARGIN_ENDED = 0.15;
 
-static RotPlan rot_plan(const int32_t *len, int64_t n, int64_t cu) {
+// (`from`: longest_of_32, made the longest of 32 and all after them here)
+static RotPlan rot_plan(std::vector<int32_t> from, int64_t cu) {
     RotPlan best;
-    std::vector<int32_t> from((size_t)((n + 31) / 32));   // longest chunk of 32 and all after them
-    for (int64_t i = (int64_t)from.size() - 1, m = 0; i >= 0; --i) {
-        m = std::max<int64_t>(m, *std::max_element(len + i * 32, len + std::min(n, i * 32 + 32)));
-        from[(size_t)i] = (int32_t)m;
-    }
+    for (size_t i = from.size() - 1; i-- > 0;) from[i] = std::max(from[i], from[i + 1]);
     for (int rt = 1; rt <= RT_TILE; ++rt) {
-        const int64_t R = 32 * rt, G = (n + R - 1) / R;
+        const int64_t G = ((int64_t)from.size() + rt - 1) / rt;
         if (G <= cu / 2) continue;
         std::vector<int32_t> longest((size_t)G);   // of the group and all after it
         for (int64_t i = 0; i < G; ++i) longest[(size_t)i] = from[(size_t)(i * rt)];
@@ -1466,11 +1482,20 @@ static int decompress_run(const sc_model *m, const uint32_t *words, const int64_
         if (!split_ok || split_force >= 0 || m->dev.n_layers < FED_MIN_LAYERS) return FedPlan{};
         return fed_plan_of(n, cu, xch_cap, fed_rt);
     };
+    // the chunks left over: split or unsplit, and fed if that is cheaper for
+    // their steps (SC_HIP_DEC_FED: in any case)
+    const int64_t left_steps = can_pair ? left_max : len_max;
     const int p_left = split_p(left);
-    const FedPlan f_left = fed_plan(left);
-    const int left_cost = f_left.heads ? f_left.cost : p_left == 8 ? DEC_SPLIT_STEP_COST_P8 : p_left == 4 ? DEC_SPLIT_STEP_COST_P4 : DEC_STEP_COST[1];
-    const bool pair = can_pair && (int64_t)std::max(0, pair_max - group_max) * DEC_STEP_COST[rt_last] <
-                                      (int64_t)left_max * left_cost;
+    int64_t left_cost = p_left == 8   ? left_steps * DEC_SPLIT_STEP_COST_P8 + SPLIT_SETUP_COST
+                        : p_left == 4 ? left_steps * DEC_SPLIT_STEP_COST_P4 + SPLIT_SETUP_COST
+                                      : left_steps * DEC_STEP_COST[1];
+    FedPlan f_left = fed_plan(left);
+    if (f_left.heads) {
+        const int64_t cost = left_steps * f_left.cost + FED_SETUP_COST + (left > 32 * XCH_MAX_GROUPS ? FED_SETUP_COST_RETRY : 0);
+        if (fed_rt || cost <= left_cost) left_cost = cost;
+        else f_left = FedPlan{};
+    }
+    const bool pair = can_pair && (int64_t)std::max(0, pair_max - group_max) * DEC_STEP_COST[rt_last] < left_cost;
     const int64_t maxlen = std::max(len_max, pair ? pair_max : 0);
     // The plan's cost against rotating launches': its launches' longest
     // chunks' steps, the pairs' or the leftover launch's.  Rotating launches
@@ -1484,18 +1509,22 @@ static int decompress_run(const sc_model *m, const uint32_t *words, const int64_
     if (m->dev.pipe == CORE_PIPE_UNI && units >= 1 && lengths_host && len_max <= (1 << 20) && !rt_cap && !plan_env &&
         !seg_env && !pair_env && !split_env && !(rot_env && std::strcmp(rot_env, "0") == 0)) {
         int64_t cost = pair ? (int64_t)std::max(0, pair_max - group_max) * DEC_STEP_COST[rt_last]
-                            : left ? (int64_t)left_max * left_cost : 0;
-        const int32_t *at = lengths_host;
+                            : left ? left_cost : 0;
+        const std::vector<int32_t> longest = longest_of_32(lengths_host, n_chunks);
+        int64_t at = 0;   // (a plan's launches are whole groups of 32)
         for (int rt : plan) {
-            const int32_t *end = at + rt * 32 * cu;
-            cost += (int64_t)std::max(0, *std::max_element(at, end)) * DEC_STEP_COST[rt];
-            at = end;
+            cost += (int64_t)longest_of(longest.data() + at, rt * cu) * DEC_STEP_COST[rt];
+            at += rt * cu;
         }
-        rot = rot_plan(lengths_host, n_chunks, cu);
-        int64_t sum = 0;
-        for (int64_t i = 0; i < n_chunks; ++i) sum += std::max(lengths_host[i], 0);
-        const double ended = len_max > 0 ? 1 - (double)sum / ((double)n_chunks * len_max) : 0;
-        if ((double)rot.cost > (double)cost * (0.98 - ROT_MARGIN_ENDED * ended)) rot.rt = 0;
+        rot = rot_plan(longest, cu);
+        if ((double)rot.cost < 0.98 * (double)cost) {
+            int64_t sum = 0;
+            for (int64_t i = 0; i < n_chunks; ++i) sum += std::max(lengths_host[i], 0);
+            const double ended = len_max > 0 ? 1 - (double)sum / ((double)n_chunks * len_max) : 0;
+            if ((double)rot.cost > (double)cost * (0.98 - ROT_MARGIN_ENDED * ended)) rot.rt = 0;
+        } else {
+            rot.rt = 0;
+        }
     }
     if (const char *log = getenv("SC_HIP_DEC_LOG"); log && std::strcmp(log, "1") == 0) {   // what is launched
         if (rot.rt) {
@@ -1505,8 +1534,8 @@ static int decompress_run(const sc_model *m, const uint32_t *words, const int64_
         } else {
             std::string rts;
             for (int rt : plan) rts += (rts.empty() ? "" : ",") + std::to_string(rt);
-            const FedPlan fl = pair ? FedPlan{} : fed_plan(left);
-            const int pl = split_p(left);
+            const FedPlan fl = pair ? FedPlan{} : f_left;
+            const int pl = p_left;
             std::fprintf(stderr, "sc_decompress_chunks: chunks %lld cu %lld plan [%s] leftover %lld %s steps %lld seg %lld fed %d+%dx%d rt %d\n",
                          (long long)n_chunks, (long long)cu, rts.c_str(), (long long)left,
                          left == 0 ? "none" : pair ? "paired" : fl.heads ? "fed launch" : pl == 8 ? "split launch p8"
@@ -1543,14 +1572,14 @@ static int decompress_run(const sc_model *m, const uint32_t *words, const int64_
             rt = 1;
             count = rest;
             grid = (unsigned)((rest + 31) / 32);
-            split = split_p(rest);
+            split = p_left;   // (rest == left)
         }
         const uint32_t *wds = words;
         const int64_t *woff = word_off + start, *toff = tok_off + start;
         const int32_t *wcnt = word_cnt + start, *len = lengths + start;
         int32_t *st = status + start;
         DecState *ds = seg > 0 ? state + start : nullptr;
-        if (const FedPlan f = tail ? fed_plan(rest) : FedPlan{}; f.heads) {
+        if (const FedPlan f = tail ? f_left : FedPlan{}; f.heads) {
             const int64_t tiles = (int64_t)f.heads * f.rt;
             hipLaunchKernelGGL(k_zero_i32, dim3(16), dim3(256), 0, s, (int32_t *)(xch + tiles * FED_SUMS),
                                tiles * FED_SYNC / 4);
@@ -1567,8 +1596,8 @@ static int decompress_run(const sc_model *m, const uint32_t *words, const int64_
                 // CUs) and decode again; larger batches never waited
                 // between workgroups before they ran fed.  Their groups that
                 // timed out are decoded again here: one launch whose
-                // workgroups look at their statuses and end (5 us beside
-                // at least 20 a step).
+                // workgroups look at their statuses and end (2 us beside 51
+                // ms at 4,000 chunks).
                 if (grid > XCH_MAX_GROUPS) {
                     launch_decompress<1>(m->dev, grid, s, wds, woff, wcnt, len, count, tokens, toff, st, nullptr, 0,
                                          INT32_MAX, 0, 0, (int32_t)grid, true);

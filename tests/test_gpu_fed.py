@@ -158,3 +158,24 @@ def test_large_fed_decode_never_reports_a_timeout(codec, monkeypatch, n, rt):
         torch.cuda.synchronize()
         assert np.array_equal(status.cpu().numpy(), want), spin
         assert np.array_equal(out.cpu().numpy()[keep], tokens[keep]), spin
+
+
+@pytest.mark.parametrize("n,longest,what", [(700, 1, "split launch p8"), (700, 8, "fed launch"), (1100, 1, "split launch p4"),
+                                            (8191, 2, "launch"), (8191, 30, "fed launch"), (4000, 1, "launch"),
+                                            (4000, 3, "fed launch")])
+def test_few_steps_run_without_feeders(codec, monkeypatch, capfd, n, longest, what):
+    """A fed launch starts 30 to 60 us later than others (its feeders load
+    layer 0): decodes of a step or two take the split or unsplit launch,
+    whichever the costs say (8,191 chunks of 1 token: 133 us fed, 88
+    unsplit)."""
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the chunk counts are for 256 CUs")
+    lengths = np.full(n, longest)
+    lengths[n // 2:] = max(longest - 1, 1)
+    tokens, lengths, words, off, cnt = _chunks(codec, lengths, n)
+    monkeypatch.setenv("SC_HIP_DEC_LOG", "1")
+    capfd.readouterr()
+    back = np.array(codec.decompress_flat(words, off, cnt, lengths)[0])
+    log = capfd.readouterr().err
+    assert f"leftover {n} {what} steps {longest} " in log, log
+    assert np.array_equal(back, tokens)
